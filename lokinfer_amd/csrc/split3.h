@@ -1,0 +1,71 @@
+// f32 products on the bf16 matrix cores. A float is the exact sum of three bf16 parts (8 + 8 + 8 significand bits):
+// h = bf16(x), m = bf16(x - h), l = x - h - m, all rounded to nearest, so |m| <= 2^-8 |x| and |l| <= 2^-16 |x|. The
+// product of two such sums is nine bf16 products; the six of order up to 2^-16 are kept,
+//   x y = l h' + h l' + m m' + m h' + h m' + h h',
+// each exact in the f32 accumulator, and the dropped three (m l', l m', l l') are below 2^-23 |x y|, 2^-26 on average
+// and of either sign. Six 32x32x16 bf16 MFMAs take 192 cycles for 16 k where eight 32x32x2 f32 MFMAs take 512, and
+// they round the accumulator six times per 16 k instead of eight: against float64, 32 x 32 dot products of N(0, 1)
+// values are off by 1.6e-7 / 4.3e-7 / 9.5e-7 (2-norm) at K = 128 / 768 / 3072, on f32 MFMAs by 2.1e-7 / 4.9e-7 / 1.0e-6.
+//
+// An infinite or NaN element, or one that rounds past the largest bf16, splits into parts of which one is NaN, and so
+// makes every output it enters NaN: kernels test their outputs for NaN and recompute such tiles on f32 MFMAs, which
+// gives the value the f32 sum has. The bf16 MFMAs flush denormal parts: elements below about 2^-110 keep fewer than
+// 24 bits.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+namespace lkd {
+
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+
+// the parts of a and b as bf16 pairs (a in the low half)
+__device__ __forceinline__ void split3(float a, float b, unsigned& h, unsigned& m, unsigned& l) {
+  h = __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2{a, b}), bf16x2));
+  const float ra = a - __uint_as_float(h << 16), rb = b - __uint_as_float(h & 0xffff0000u);
+  m = __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2{ra, rb}), bf16x2));
+  l = __builtin_bit_cast(unsigned, __builtin_convertvector(
+                                       (f32x2{ra - __uint_as_float(m << 16), rb - __uint_as_float(m & 0xffff0000u)}),
+                                       bf16x2));
+}
+
+__device__ __forceinline__ void split3(f32x4 x, u32x2& h, u32x2& m, u32x2& l) {
+  unsigned a[3], b[3];
+  split3(x[0], x[1], a[0], a[1], a[2]);
+  split3(x[2], x[3], b[0], b[1], b[2]);
+  h = u32x2{a[0], b[0]};
+  m = u32x2{a[1], b[1]};
+  l = u32x2{a[2], b[2]};
+}
+
+// An operand fragment of a 32x32x16 MFMA (8 consecutive k of one row or column per lane) in its three parts.
+struct Frag3 {
+  bf16x8 h, m, l;
+};
+
+__device__ __forceinline__ Frag3 split3(f32x4 x0, f32x4 x1) {
+  u32x2 h0, m0, l0, h1, m1, l1;
+  split3(x0, h0, m0, l0);
+  split3(x1, h1, m1, l1);
+  return Frag3{__builtin_bit_cast(bf16x8, (u32x4{h0[0], h0[1], h1[0], h1[1]})),
+               __builtin_bit_cast(bf16x8, (u32x4{m0[0], m0[1], m1[0], m1[1]})),
+               __builtin_bit_cast(bf16x8, (u32x4{l0[0], l0[1], l1[0], l1[1]}))};
+}
+
+// acc += a b over 16 k, the smallest products first
+__device__ __forceinline__ f32x16 mfma3(const Frag3& a, const Frag3& b, f32x16 acc) {
+  acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.l, b.h, acc, 0, 0, 0);
+  acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.h, b.l, acc, 0, 0, 0);
+  acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.m, b.m, acc, 0, 0, 0);
+  acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.m, b.h, acc, 0, 0, 0);
+  acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.h, b.m, acc, 0, 0, 0);
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.h, b.h, acc, 0, 0, 0);
+}
+
+}  // namespace lkd

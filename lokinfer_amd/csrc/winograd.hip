@@ -11,14 +11,14 @@
 // The same kernels run this backend's Kokoro graph wherever their grid fills the chip (the generator's resblock
 // and noise convs, the decoder's wide convs, conv_post).
 //
-// wino_mm: one workgroup per (64 output channels, 64 tiles, residue); 4 waves in 2 x 2, each 32 tiles x 32
-// channels. Steps = points x 16-channel chunks; per step the V rows of the workgroup's tiles (+ N - 1 for the
-// group shift) are staged [row][4 slots] (swizzled by (row >> 2) & 3) and U's N x 16 rows k-major; the point's
-// GEMM accumulates over the groups with the A rows shifted by g, and after a point's last chunk AT[j, xi] folds
-// it into the M output accumulators. Small grids split the steps over workgroups (split-K) and sum the partial
-// rows in winoSplitReduceKernel (statistics then from the channel-stats kernel).
+// wino_mm: one workgroup per (64 output channels, 64 tiles, residue); 4 waves in 2 x 2, each 32 tiles x 32 channels.
+// Steps = points x 16-channel chunks; the point's GEMM accumulates over the groups with the A rows shifted by g, and
+// after a point's last chunk AT[j, xi] folds it into the M output accumulators. Small grids split the steps over
+// workgroups (split-K) and sum the partial rows in winoSplitReduceKernel (statistics then from the channel-stats
+// kernel).
 #include "common.h"
 #include "lokinfer_hip.h"
+#include "split3.h"
 
 #include <algorithm>
 #include <cstdint>
@@ -29,7 +29,6 @@ int residueStats(const float* x, float* st, int64_t l, int64_t c, int d, int64_t
 
 namespace lkd {
 
-typedef float v16w __attribute__((ext_vector_type(16)));
 typedef float v4w __attribute__((ext_vector_type(4)));
 
 constexpr int kWinoRows = 128;  // output rows per statistics chunk
@@ -106,6 +105,16 @@ __global__ __launch_bounds__(256) void winoTfKernel(const float* __restrict__ x,
   }
 }
 
+// A raw buffer resource over `bytes` bytes from p, both the same in every lane (read from the first, so that they are
+// held in scalar registers).
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t uniformRsrc(const void* p, unsigned bytes) {
+  const uint64_t a = reinterpret_cast<uint64_t>(p);
+  const uint64_t lo = static_cast<unsigned>(__builtin_amdgcn_readfirstlane(static_cast<int>(a)));
+  const uint64_t hi = static_cast<unsigned>(__builtin_amdgcn_readfirstlane(static_cast<int>(a >> 32)));
+  return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>(hi << 32 | lo), 0,
+                                           __builtin_amdgcn_readfirstlane(static_cast<int>(bytes)), 0x00020000);
+}
+
 struct WinoMmArgs {
   const float* v;
   const float* u;
@@ -120,33 +129,51 @@ struct WinoMmArgs {
   float scale;
 };
 
-// OCC workgroups per CU. M = 4 at OCC = 3 fits 168 VGPRs (the few spills the bound costs sit before the step loop
-// and in the epilogue): on grids of more than two workgroups per CU a third wave per SIMD keeps the matrix pipe fed
-// through the other waves' barriers and LDS stores (K = 11 roofline launch 0.574 -> 0.599 of peak); smaller grids
-// leave the third slot empty and run the unconstrained OCC = 2 form (176 VGPRs), which is 0.5% faster there.
+// The three bf16 parts of 8 values, in r[0 .. 2], become the values themselves, in r[0] and r[1].
+__device__ __forceinline__ void joinParts(f32x4 (&r)[3]) {
+  const u32x4 h = __builtin_bit_cast(u32x4, r[0]), m = __builtin_bit_cast(u32x4, r[1]);
+  const u32x4 l = __builtin_bit_cast(u32x4, r[2]);
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int o = 0; o < 2; ++o) {
+      const auto f = [&](unsigned x) { return __uint_as_float(o ? x & 0xffff0000u : x << 16); };
+      r[i >> 1][2 * (i & 1) + o] = (f(h[i]) + f(m[i])) + f(l[i]);
+    }
+}
+
+// MFMA-bound: the products run on the bf16 matrix cores as three-part splits (split3.h), 6 N S MFMAs of 32 cycles per
+// wave and step of S 16-channel chunks, at three workgroups per CU (at most 168 registers): the y accumulators leave
+// room for one 32 x 32 block per wave, and it takes three waves per SIMD to cover a step's loads, LDS stores and
+// barrier (two blocks per wave at two waves per SIMD ran 5 - 35% slower).
 //
-// S: 16-channel sub-chunks per step (one tap group only). A step of one tap group and 16 channels is 8 MFMAs per
-// wave, too few to cover the step's fixed costs (barrier, staging, the first operand reads); S sub-chunks make it
-// 8 S MFMAs. Sub-chunk s of the step's 16 S channels has its own A plane, laid out as a 16-channel step's.
+// A: the step's V rows (64 tiles + N - 1 for the group shift) are split once while staging and held in LDS as three bf16
+// planes, [row][2 halves of 8 channels], half swizzled by (row >> 3) & 1 so that 16 lanes of a 16-byte read cover all 64
+// banks. B bypasses LDS: a wave's fragment (16 k x 32 columns) comes straight from U, one step ahead, in coalesced
+// 16-byte loads.
 //
-// UT: U given tiled (ops u_layout = 1), Ut [A, Co / 64, (Ci / 16) N 4 64 4]: per point and 64-column block, for
-// each 16-channel chunk and tap group the 16 x 64 slab stored k-quad-major, [k4][col][4] (U row g Ci + 16 c + 4 k4 + q,
-// column 64 cb + col). A step's U is then one contiguous run, staged with coalesced 16-byte loads straight into
-// the LDS order Bs[e * 4 + k4][col] (e = g S + s), and a wave fetches an operand set's B fragments for eight MFMAs
-// with two 16-byte reads: 4 N S reads per step in all, few enough for the LDS counter to wait on each read
-// separately (with U k-major, the 16 N S + 2 N S reads of a step exceed it). The same MFMAs in the same order, so
-// the same bits.
-template <int M, int A, int N, int OCC = 2, int S = 1, bool UT = false>
-__global__ __launch_bounds__(256, OCC) void winoMmKernel(WinoMmArgs p) {
-  static_assert(S == 1 || N == 1, "sub-chunks only for one tap group");
-  constexpr int TT = 64;              // tiles per workgroup
-  constexpr int ROWS = TT + N - 1;    // staged V rows (group shift)
-  constexpr int LDB = 64 + 8;         // k-major U rows: the two lane halves read 4 rows = 32 banks apart
-  constexpr int AQ = ROWS * 4;
-  constexpr int AS1 = (AQ + 255) / 256;  // staging float4s per thread and sub-chunk
-  constexpr int AS = S * AS1;
-  __shared__ v4w As[2][AS * 256];  // rows past ROWS: every thread stores, so no store sits behind a branch
-  __shared__ float Bs[2][UT ? N * S * 16 * 64 : N * S * 16 * LDB];
+// Measured (U split, graph replay), against the f32 MFMA form of this kernel, which reached 110 of 157 TFLOP/s and could
+// not overlap its vector instructions with its MFMAs: L = 293281, 128 -> 128 channels, K = 11 d = 5 456 -> 333 us,
+// K = 7 d = 3 335 -> 249 us, K = 3 with residual 254 -> 161 us; L = 48880, 256 -> 256, K = 11 d = 3 304 -> 213 us; L =
+// 5740, 256 -> 256, K = 7 d = 3 64 -> 49 us. Without the V staging the first takes 269 us, without the U loads 301, with
+// neither 223, and its bf16 MFMAs alone 148 (2.05 PFLOP/s).
+//
+// UL, the layout of U:
+//   0  U [A, N Ci, Co]: eight 4-byte loads per fragment, split before its MFMAs;
+//   1  tiled (ops u_layout = 1), Ut [A, Co / 64, (Ci / 16) N 4 64 4]: per point and 64-column block, for each 16-channel
+//      chunk and tap group the 16 x 64 slab stored k-quad-major, [k4][col][4] (U row g Ci + 16 c + 4 k4 + q, column
+//      64 cb + col): two 16-byte loads;
+//   2  split (ops u_layout = 2), Us [A, Co / 64, 2, Ci / 16, N, 3, 64, 8] bf16: per 32-column half, chunk and group the
+//      three parts (h, m, l) in fragment order, lane 32 lk + lr holding k = 8 lk .. 8 lk + 7 of column lr: three 16-byte
+//      loads and nothing to split.
+template <int M, int A, int N, int S, int UL>
+__global__ __launch_bounds__(256, 3) void winoMmKernel(WinoMmArgs p) {
+  constexpr int TT = 64;            // tiles per workgroup
+  constexpr int ROWS = TT + N - 1;  // staged V rows (group shift)
+  constexpr int E = N * S;          // B fragments of a step: e = N (chunk) + (tap group)
+  using Stage = u32x4[S][3][ROWS * 2];
+  using RawB = f32x4[UL == 2 ? 3 : 2];
+  __shared__ Stage As0, As1;  // two objects, so that the compiler sees that a step's stores and reads never meet
   __shared__ float red[2][64];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave >> 1, wn = wave & 1, lr = lane & 31, lk = lane >> 5;
@@ -157,206 +184,311 @@ __global__ __launch_bounds__(256, OCC) void winoMmKernel(WinoMmArgs p) {
   const int64_t t0 = static_cast<int64_t>(wk.y) * TT;
   if (t0 * M >= lor) return;
   const int64_t c0 = static_cast<int64_t>(wk.x) * 64;
-  const int chunks = static_cast<int>(p.ci / (16 * S));
+  const int ci = static_cast<int>(p.ci), co = static_cast<int>(p.co);
+  const int chunks = ci / (16 * S);
   const int steps = A * chunks;
   // split-K: this workgroup runs steps [sb, se) of the point-major step sequence; a point cut by the range is
   // folded with AT at the range's end, and AT is linear, so the splits' outputs sum to the full one
   const int sb = static_cast<int>(static_cast<int64_t>(steps) * sp / p.split);
   const int se = static_cast<int>(static_cast<int64_t>(steps) * (sp + 1) / p.split);
-  const int nsteps = se - sb;
-  const int64_t nci = static_cast<int64_t>(N) * p.ci;
-
-  // staging: A rows (S planes of ROWS x 4 slots) over 256 threads, U (N S 16 rows x 16 float4) over 256 threads
-  constexpr int BQ = N * S * 16 * 16;
-  constexpr int BSL = BQ / 256;
-  // two register sets: step t's operands live in set t & 1, loaded two steps ahead of their LDS store
-  v4w ra0[AS], rb0[BSL], ra1[AS], rb1[BSL];
-  auto gload = [&](int s, v4w(&ra)[AS], v4w(&rb)[BSL]) {
-    const int xi = s / chunks, ch = s - xi * chunks;
-    const float* vx =
-        p.v + (static_cast<int64_t>(rho) * A + xi) * p.rmax * p.ci + static_cast<int64_t>(ch) * 16 * S;
-#pragma unroll
-    for (int i = 0; i < AS; ++i) {
-      const int idx = tid + 256 * (i % AS1);
-      const int row = min(idx >> 2, ROWS - 1), slot = idx & 3;
-      const int64_t t = min<int64_t>(t0 + row, p.rmax - 1);  // rows past rmax only feed tiles never stored
-      ra[i] = *reinterpret_cast<const v4w*>(vx + t * p.ci + 16 * (i / AS1) + 4 * slot);
-    }
-    const float* ux = UT ? p.u + (static_cast<int64_t>(xi) * (p.co / 64) + c0 / 64) * nci * 64 +
-                               static_cast<int64_t>(ch) * (N * S * 1024)
-                         : p.u + static_cast<int64_t>(xi) * nci * p.co + c0;
-#pragma unroll
-    for (int i = 0; i < BSL; ++i) {
-      const int idx = tid + 256 * i;
-      if constexpr (UT) {  // the step's slab, in the LDS order
-        rb[i] = *reinterpret_cast<const v4w*>(ux + 4 * idx);
-      } else {
-        const int c4 = idx & 15, gk = idx >> 4, g = gk / (16 * S), k = gk % (16 * S);
-        rb[i] =
-            *reinterpret_cast<const v4w*>(ux + (static_cast<int64_t>(g) * p.ci + ch * 16 * S + k) * p.co + 4 * c4);
-      }
-    }
-  };
-  auto sstore = [&](int buf, const v4w(&ra)[AS], const v4w(&rb)[BSL]) {
-#pragma unroll
-    for (int i = 0; i < AS; ++i) {
-      const int idx = tid + 256 * (i % AS1);
-      const int row = idx >> 2, slot = idx & 3;
-      As[buf][(i / AS1) * AS1 * 256 + row * 4 + (slot ^ ((row >> 2) & 3))] = ra[i];
-    }
-#pragma unroll
-    for (int i = 0; i < BSL; ++i) {
-      const int idx = tid + 256 * i;
-      if constexpr (UT) {
-        *reinterpret_cast<v4w*>(&Bs[buf][4 * idx]) = rb[i];
-      } else {
-        const int c4 = idx & 15, gk = idx >> 4;
-        *reinterpret_cast<v4w*>(&Bs[buf][gk * LDB + 4 * c4]) = rb[i];
-      }
-    }
-  };
-
-  v16w acc, y[M];
-#pragma unroll
-  for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
-#pragma unroll
-  for (int j = 0; j < M; ++j)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) y[j][r] = 0.0f;
-
+  const int64_t nci = static_cast<int64_t>(N) * ci;
   const int arow = 32 * wm + lr, bcol = 32 * wn + lr;
-  // one step: MFMAs on LDS buffer s & 1; loads step s + 2 into (lra, lrb) = set s & 1 (its step s is already in
-  // LDS), stores step s + 1 from (sra, srb) = set (s + 1) & 1 into the other buffer
-  auto step = [&](int sl, v4w(&lra)[AS], v4w(&lrb)[BSL], const v4w(&sra)[AS], const v4w(&srb)[BSL]) {
-    const int buf = sl & 1, s = sb + sl;
-    const int xi = s / chunks, ch = s - xi * chunks;
-    // operand sets (tap group g, sub-chunk s) = e = g S + s
-    v4w af[N * S][2];
-    float bq[N * S][2][4];
+
+  // Operand addresses are a uniform pointer, advanced per step by scalar arithmetic, plus a 32-bit per-lane offset.
+  // V: rows past rmax (they only feed tiles never stored) read the last one.
+  auto vAt = [&](int xi, int ch) {
+    return p.v + ((static_cast<int64_t>(rho) * A + xi) * p.rmax + t0) * ci + static_cast<int64_t>(ch) * 16 * S;
+  };
+  constexpr int kSet = UL == 0 ? 0 : UL == 1 ? 1024 : 768;  // floats of a fragment's slab (UL 2: of its 32-column half)
+  auto uAt = [&](int xi, int ch) {
+    if constexpr (UL == 0) return p.u + (static_cast<int64_t>(xi) * nci + ch * 16 * S) * co + c0;
+    return p.u + (static_cast<int64_t>(xi) * (co / 64) + c0 / 64) * nci * (UL == 1 ? 64 : 96) +
+           static_cast<int64_t>(ch) * E * kSet;
+  };
+  // from one step's operands to the next one's, and what a new point adds
+  const int64_t vWrap = (p.rmax - 1) * ci;
+  const int64_t uStep = UL == 0 ? static_cast<int64_t>(16 * S) * co : E * kSet;
+  const int64_t uWrap = UL == 0   ? (nci - ci) * co
+                        : UL == 1 ? (co / 64 - 1) * nci * 64
+                                  : (co / 64) * nci * 96 - nci * 48;
+  auto vRow = [&](int row) { return static_cast<unsigned>(min<int64_t>(row, p.rmax - 1 - t0)) * ci; };
+  // Raw V of a step: a float4 of row tid / 4 (quad tid % 4) per chunk, and one float of the N - 1 extra rows, held by
+  // every 16 (N - 1) S threads alike.
+  struct RawA {
+    f32x4 v[S];
+    float x;
+  } ra0, ra1;
+  const int srow = tid >> 2, squad = tid & 3;
+  constexpr int XN = N > 1 ? N - 1 : 1;
+  const int xch = tid & 15, xrow = TT + (tid >> 4) % XN, xsub = (tid >> 4) / XN % S;
+  const unsigned aoff = vRow(srow) + 4 * squad, xoff = vRow(xrow) + 16 * xsub + xch;
+  const unsigned boff = UL == 0   ? 8 * lk * co + bcol
+                        : UL == 1 ? (2 * lk * 64 + bcol) * 4
+                                  : static_cast<unsigned>(wn * nci * 48) + lane * 4;
+  auto loadA = [&](const float* vx, RawA& ra) {
 #pragma unroll
-    for (int e = 0; e < N * S; ++e) {
-      const int row = arow + e / S;
-      const int plane = (e % S) * AS1 * 256;
+    for (int i = 0; i < S; ++i) ra.v[i] = *reinterpret_cast<const f32x4*>(vx + 16 * i + aoff);
+    if constexpr (N > 1) ra.x = vx[xoff];
+  };
+  auto storeA = [&](Stage& As, const RawA& ra) {
 #pragma unroll
-      for (int h = 0; h < 2; ++h) af[e][h] = As[buf][plane + row * 4 + ((2 * h + lk) ^ ((row >> 2) & 3))];
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        if constexpr (UT) {
-          const v4w b4 = *reinterpret_cast<const v4w*>(&Bs[buf][((e * 4 + 2 * h + lk) * 64 + bcol) * 4]);
-#pragma unroll
-          for (int q = 0; q < 4; ++q) bq[e][h][q] = b4[q];
-        } else {
-#pragma unroll
-          for (int q = 0; q < 4; ++q) bq[e][h][q] = Bs[buf][(e * 16 + 8 * h + 4 * lk + q) * LDB + bcol];
-        }
-      }
+    for (int i = 0; i < S; ++i) {
+      u32x2 h, m, l;
+      split3(ra.v[i], h, m, l);
+      const int s2 = 4 * srow + 2 * ((squad >> 1) ^ ((srow >> 3) & 1)) + (squad & 1);
+      reinterpret_cast<u32x2*>(As[i][0])[s2] = h;
+      reinterpret_cast<u32x2*>(As[i][1])[s2] = m;
+      reinterpret_cast<u32x2*>(As[i][2])[s2] = l;
     }
-    // unconditional (the last two steps reload the final step), so the wait before each LDS store counts only
-    // the loads of the set it stores and never the ones just issued
-    gload(min(s + 2, se - 1), lra, lrb);
-#pragma unroll
-    for (int e = 0; e < N * S; ++e)
+    if constexpr (N > 1) {
+      unsigned h, m, l;
+      split3(ra.x, 0.0f, h, m, l);
+      const int s8 = 8 * (xrow * 2 + ((xch >> 3) ^ ((xrow >> 3) & 1))) + (xch & 7);
+      reinterpret_cast<unsigned short*>(As[xsub][0])[s8] = static_cast<unsigned short>(h);
+      reinterpret_cast<unsigned short*>(As[xsub][1])[s8] = static_cast<unsigned short>(m);
+      reinterpret_cast<unsigned short*>(As[xsub][2])[s8] = static_cast<unsigned short>(l);
+    }
+  };
+  // channels 8 lk .. 8 lk + 7 of fragment e's 16, column c0 + bcol
+  auto loadB = [&](const float* ux, int e, RawB& r) {
+    if constexpr (UL == 0) {
+      const float* ue = ux + (static_cast<int64_t>(e % N) * ci + (e / N) * 16) * co;
 #pragma unroll
       for (int h = 0; h < 2; ++h)
 #pragma unroll
-        for (int q = 0; q < 4; ++q) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(af[e][h][q], bq[e][h][q], acc, 0, 0, 0);
-    if (ch == chunks - 1 || s == se - 1) {  // the point (or this split's part of it) is complete: fold it
+        for (int q = 0; q < 4; ++q) r[h][q] = ue[(4 * h + q) * co + boff];
+    } else {
 #pragma unroll
-      for (int j = 0; j < M; ++j) {
-        const float at = p.tr[A * A + j * A + xi];
-        y[j] += at * acc;
-      }
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
+      for (int h = 0; h < (UL == 1 ? 2 : 3); ++h)
+        r[h] = *reinterpret_cast<const f32x4*>(ux + e * kSet + h * 256 + boff);
     }
-    sstore(buf ^ 1, sra, srb);  // after the last step, into a buffer nothing reads
-    __syncthreads();
+  };
+  auto partsB = [&](const RawB& r) {
+    if constexpr (UL == 2)
+      return Frag3{__builtin_bit_cast(bf16x8, r[0]), __builtin_bit_cast(bf16x8, r[1]),
+                   __builtin_bit_cast(bf16x8, r[2])};
+    else
+      return split3(r[0], r[1]);
   };
 
-  gload(sb, ra0, rb0);
-  sstore(0, ra0, rb0);
-  gload(min(sb + 1, se - 1), ra1, rb1);
+  f32x16 acc;
+  float y[M][16];
+  auto clear = [&](auto& x) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) x[r] = 0.0f;
+  };
+  // a finished point (or this split's part of it) folds into the output rows
+  auto fold = [&](int xi) {
+#pragma unroll
+    for (int j = 0; j < M; ++j) {
+      const float at = p.tr[A * A + j * A + xi];
+#pragma unroll
+      for (int r = 0; r < 16; ++r) y[j][r] += at * acc[r];
+    }
+    clear(acc);
+  };
+  clear(acc);
+#pragma unroll
+  for (int j = 0; j < M; ++j) clear(y[j]);
+
+  // A step computes from one LDS buffer. Its first work is to split and store the next step's V rows, loaded two steps
+  // earlier, into the other one, and to load those of the step after the next but one into the same registers (V comes
+  // from HBM). Past the last step the operands of the last are loaded again. cv, cu: chunk of the step whose V / U
+  // pointer is vp / up; xs, cs: point and chunk of the step being computed.
+  int xs = sb / chunks, cs = sb - xs * chunks, cv = cs, cu = cs;
+  const float *vp = vAt(xs, cs), *up = uAt(xs, cs);
+  auto nextV = [&](bool more) {
+    const bool wrap = cv + 1 == chunks;
+    vp += more ? 16 * S + (wrap ? vWrap : 0) : 0;
+    cv = more ? (wrap ? 0 : cv + 1) : cv;
+  };
+  auto nextU = [&](bool more) {
+    const bool wrap = cu + 1 == chunks;
+    up += more ? uStep + (wrap ? uWrap : 0) : 0;
+    cu = more ? (wrap ? 0 : cu + 1) : cu;
+  };
+  RawB rb[E];
+  loadA(vp, ra0);
+  nextV(sb + 1 < se);
+  loadA(vp, ra1);
+#pragma unroll
+  for (int e = 0; e < E; ++e) loadB(up, e, rb[e]);
+  storeA(As0, ra0);
+  nextV(sb + 2 < se);
+  loadA(vp, ra0);
   __syncthreads();
-  // pairs of steps with no branch inside, so every loop edge carries the same outstanding loads; an odd last
-  // step is peeled
-  int sl = 0;
-  for (; sl + 1 < nsteps; sl += 2) {
-    step(sl, ra0, rb0, ra1, rb1);
-    step(sl + 1, ra1, rb1, ra0, rb0);
-  }
-  if (sl < nsteps) step(sl, ra0, rb0, ra1, rb1);
-
-  if (p.split > 1) {  // raw partial rows; bias, residual, scale and statistics come in the reduction
-    float* pp = p.part + static_cast<int64_t>(sp) * p.lo * p.co;
+  auto step = [&](int s, Stage& As, Stage& other, RawA& ra) {
+    storeA(other, ra);
+    nextV(s + 3 < se);
+    nextU(s + 1 < se);
+    loadA(vp, ra);
+    auto fragA = [&](int e) {
+      const int row = arow + e % N, slot = row * 2 + (lk ^ ((row >> 3) & 1));
+      return Frag3{__builtin_bit_cast(bf16x8, As[e / N][0][slot]), __builtin_bit_cast(bf16x8, As[e / N][1][slot]),
+                   __builtin_bit_cast(bf16x8, As[e / N][2][slot])};
+    };
+    Frag3 af = fragA(0);
 #pragma unroll
-    for (int j = 0; j < M; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int64_t uo = (t0 + 32 * wm + 8 * (r >> 2) + 4 * lk + (r & 3)) * M + j;
-        if (uo < lor) pp[(rho + uo * d) * p.co + c0 + 32 * wn + lr] = y[j][r];
-      }
-    return;
+    for (int e = 0; e < E; ++e) {
+      const Frag3 bf = partsB(rb[e]), cur = af;
+      if (e + 1 < E) af = fragA(e + 1);  // the next fragment's reads cover this one's MFMAs
+      acc = mfma3(cur, bf, acc);
+      loadB(up, e, rb[e]);  // the next step's
+    }
+    const bool wrap = cs + 1 == chunks;
+    if (wrap || s == se - 1) fold(xs);
+    cs = wrap ? 0 : cs + 1;
+    xs += wrap;
+    __syncthreads();
+  };
+  int s = sb;
+  for (; s + 1 < se; s += 2) {
+    step(s, As0, As1, ra1);
+    step(s + 1, As1, As0, ra0);
   }
+  if (s < se) step(s, As0, As1, ra1);
 
-  // epilogue: register r = tile t0 + 32 wm + 8 (r / 4) + 4 lk + r % 4, channel c0 + bcol
-  const int64_t col = c0 + bcol;
-  const float bias = p.bias[col];
+  // a non-finite or overflowing operand leaves NaN in every output it enters: such a wave runs its steps again on
+  // f32 MFMAs, operands straight from memory
+  float nan = 0.0f;
 #pragma unroll
   for (int j = 0; j < M; ++j)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int64_t t = t0 + 32 * wm + 8 * (r >> 2) + 4 * lk + (r & 3);
-      const int64_t uo = t * M + j;
-      float o = y[j][r] + bias;
-      if (p.res && uo < lor) o += p.res[(rho + uo * d) * p.co + col];
-      o *= p.scale;
-      y[j][r] = o;
-      if (uo < lor) p.out[(rho + uo * d) * p.co + col] = o;
+    for (int r = 0; r < 16; ++r) nan += y[j][r];
+  if (__any(nan != nan)) {
+#pragma unroll
+    for (int j = 0; j < M; ++j) clear(y[j]);
+#pragma unroll 1
+    for (int f = sb; f < se; ++f) {
+      const int xf = f / chunks, cf = f - xf * chunks;
+      const float *vf = vAt(xf, cf), *uf = uAt(xf, cf);
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+        RawB bq;
+        loadB(uf, e, bq);
+        if constexpr (UL == 2) joinParts(bq);
+        const float* vr = vf + vRow(arow + e % N) + 16 * (e / N) + 8 * lk;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const f32x4 aq = *reinterpret_cast<const f32x4*>(vr + 4 * h);
+#pragma unroll
+          for (int q = 0; q < 4; ++q) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(aq[q], bq[h][q], acc, 0, 0, 0);
+        }
+      }
+      if (cf == chunks - 1 || f == se - 1) fold(xf);
     }
+  }
+
+  // Register r = tile tb0 + 8 (r / 4) + 4 lk + r % 4, channel c0 + bcol. Output rows go through buffer resources that
+  // end with the tensor (a row past the residue class is past the tensor): loads there give 0 and stores are dropped,
+  // with no branch per element. One resource per 8-tile row group keeps the lane offsets in 32 bits.
+  const int64_t tb0 = t0 + 32 * __builtin_amdgcn_readfirstlane(wm);
+  const int left = static_cast<int>(min<int64_t>(lor - tb0 * M, 32 * M)) - 4 * lk * M;  // output rows from this lane's
+  auto orow = [&](int j, int r) { return (8 * (r >> 2) + (r & 3)) * M + j; };
+  const unsigned rowBytes = static_cast<unsigned>(d * co) * 4;
+  const unsigned ooff = 4 * lk * M * rowBytes + static_cast<unsigned>(c0 + bcol) * 4;
+  auto rows = [&](const float* base, int rg) {  // the 8-tile group rg
+    const int64_t first = rho + (tb0 + 8 * rg) * M * d;
+    const int64_t bytes = base ? min<int64_t>(max<int64_t>(p.lo - first, 0) * co * 4, 0xfffffff0) : 0;
+    return uniformRsrc(base + (bytes ? first * co : 0), static_cast<unsigned>(bytes));
+  };
+  auto store = [&](float* base) {
+#pragma unroll
+    for (int rg = 0; rg < 4; ++rg) {
+      const auto rs = rows(base, rg);
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int j = 0; j < M; ++j)
+          __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(y[j][4 * rg + r]), rs, ooff + (r * M + j) * rowBytes, 0,
+                                                0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  if (p.split > 1) {  // raw partial rows; bias, residual, scale and statistics come in the reduction
+    store(p.part + static_cast<int64_t>(sp) * p.lo * co);
+    return;
+  }
+
+  const float bias = p.bias[c0 + bcol];
+  // every residual load before the first store; no residual: an empty resource, whose loads give 0
+  const __amdgpu_buffer_rsrc_t rs[4] = {rows(p.res, 0), rows(p.res, 1), rows(p.res, 2), rows(p.res, 3)};
+#pragma unroll
+  for (int j = 0; j < M; ++j) {
+    float rv[16];
+#pragma unroll
+    for (int r = 0; r < 16; ++r)
+      rv[r] = __uint_as_float(
+          __builtin_amdgcn_raw_buffer_load_b32(rs[r >> 2], ooff + ((r & 3) * M + j) * rowBytes, 0, 0));
+#pragma unroll
+    for (int r = 0; r < 16; ++r) y[j][r] = ((y[j][r] + bias) + rv[r]) * p.scale;
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  store(p.out);
   if (p.stats) {
-    // chunks of 128 rows of this residue class: M = 4: 32 tiles = one wave row (chunk 2 by + wm), reduced in the
-    // wave; M = 2: 64 tiles = the workgroup (chunk by), the two wave rows combined through LDS.
+    // chunks of 128 rows of this residue class. M = 4: 32 tiles, one wave row, reduced in the wave; M = 2: the
+    // workgroup's 64 tiles, the two wave rows combined through LDS.
     constexpr int TPC = kWinoRows / M;  // tiles per chunk
-    const int64_t chunk = (t0 + 32 * wm) / TPC;
-    const int64_t cbase = chunk * kWinoRows;
-    const float nrows = static_cast<float>(min<int64_t>(kWinoRows, lor - cbase));
-    float s1 = 0.0f;
+    const int64_t chunk = tb0 / TPC;
+    const float nrows = static_cast<float>(min<int64_t>(kWinoRows, lor - chunk * kWinoRows));
+    const bool whole = lor - tb0 * M >= 32 * M;
+    auto rowSum = [&](auto term) {
+      float t = 0.0f;
+      if (whole) {
 #pragma unroll
-    for (int j = 0; j < M; ++j)
+        for (int j = 0; j < M; ++j)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int64_t uo = (t0 + 32 * wm + 8 * (r >> 2) + 4 * lk + (r & 3)) * M + j;
-        if (uo < lor) s1 += y[j][r];
+          for (int r = 0; r < 16; ++r) t += term(y[j][r]);
+      } else {
+#pragma unroll
+        for (int j = 0; j < M; ++j)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) t += orow(j, r) < left ? term(y[j][r]) : 0.0f;
       }
-    s1 += __shfl_xor(s1, 32, 64);
-    if constexpr (TPC == 64) {
-      if (lk == 0) red[wm][bcol] = s1;
-      __syncthreads();
-      s1 = red[0][bcol] + red[1][bcol];
-      __syncthreads();
-    }
-    const float mean = s1 / nrows;
-    float s2 = 0.0f;
-#pragma unroll
-    for (int j = 0; j < M; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int64_t uo = (t0 + 32 * wm + 8 * (r >> 2) + 4 * lk + (r & 3)) * M + j;
-        const float dv = y[j][r] - mean;
-        if (uo < lor) s2 += dv * dv;
+      t += __shfl_xor(t, 32, 64);
+      if constexpr (TPC == 64) {
+        __syncthreads();
+        if (lk == 0) red[wm][bcol] = t;
+        __syncthreads();
+        t = red[0][bcol] + red[1][bcol];
       }
-    s2 += __shfl_xor(s2, 32, 64);
-    if constexpr (TPC == 64) {
-      if (lk == 0) red[wm][bcol] = s2;
-      __syncthreads();
-      s2 = red[0][bcol] + red[1][bcol];
-    }
-    const bool writer = lk == 0 && (TPC == 32 || wm == 0) && nrows > 0.0f;
-    if (writer) {
-      float* st = p.stats + ((static_cast<int64_t>(rho) * p.chunks + chunk) * p.co + col) * 2;
+      return t;
+    };
+    const float mean = rowSum([](float v) { return v; }) / nrows;
+    const float m2 = rowSum([&](float v) { return (v - mean) * (v - mean); });
+    if (lk == 0 && (TPC == 32 || wm == 0) && nrows > 0.0f) {
+      float* st = p.stats + ((static_cast<int64_t>(rho) * p.chunks + chunk) * co + c0 + bcol) * 2;
       st[0] = mean;
-      st[1] = s2;
+      st[1] = m2;
     }
+  }
+}
+
+// Ut (u_layout 1) -> Us (u_layout 2), a fragment's 8 values per thread. Parts of a value that would round past the
+// largest bf16 are cut instead of rounded, infinities and NaN are h alone, so that the parts always sum to the value.
+__global__ __launch_bounds__(256) void winoSplitUKernel(const float* __restrict__ ut, u32x4* __restrict__ us,
+                                                       int64_t slabs, int64_t sets) {
+  const int64_t total = slabs * sets * 128;
+  for (int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < total;
+       i += static_cast<int64_t>(gridDim.x) * blockDim.x) {
+    const int lane = static_cast<int>(i & 63), half = static_cast<int>(i >> 6) & 1;
+    const int64_t set = (i >> 7) % sets, slab = (i >> 7) / sets;
+    const float* src = ut + (slab * sets + set) * 1024 + ((lane >> 5) * 128 + half * 32 + (lane & 31)) * 4;
+    u32x4 parts[3];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      float rest = src[(k >> 2) * 256 + (k & 3)];
+      const bool finite = fabsf(rest) <= 3.40282347e38f, cut = fabsf(rest) >= 3.38953139e38f;
+#pragma unroll
+      for (int q = 0; q < 3; ++q) {
+        const unsigned b = __float_as_uint(rest);
+        const unsigned part = (cut || !finite ? b : b + 0x7fff + ((b >> 16) & 1)) >> 16;
+        rest = finite ? rest - __uint_as_float(part << 16) : 0.0f;
+        parts[q][k >> 1] = k & 1 ? parts[q][k >> 1] | part << 16 : part;
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < 3; ++q) us[((slab * 2 + half) * sets + set) * 192 + q * 64 + lane] = parts[q];
   }
 }
 
@@ -421,7 +553,7 @@ int lk_hip_wino_tf_lc_f32(const float* x, const float* tr, const float* affine, 
 
 namespace {
 
-template <bool UT>
+template <int UL>
 int winoMm(const float* v, const float* u, const float* bias, const float* res, float* out, const float* tr,
            float* stats, int64_t v_rows, int64_t ci, int64_t co, int64_t lo, int dilation, int groups, int kernel,
            int tile, float scale, void* workspace, int64_t workspace_bytes, void* stream) {
@@ -437,9 +569,11 @@ int winoMm(const float* v, const float* u, const float* bias, const float* res, 
   // measured slower than no split on MI355X: the partial rows' round trip and the second launch outweigh the extra
   // workgroups; so did splits up to three workgroups per CU at 16 steps), partials in the workspace past its 64 KiB
   // counter area
+  if (static_cast<int64_t>(dilation) * co >= int64_t{1} << 25) return 1;  // 32 output rows within 32-bit offsets
   const int64_t base = (co / 64) * ((tiles + 63) / 64) * dilation;
   const int steps = a * static_cast<int>(ci / 16);  // in 16-channel units
-  // one tap group: 48 or 32 channels per pipeline step where they divide Ci
+  // one tap group: 48 or 32 channels per pipeline step where they divide Ci (with more groups the second chunk's
+  // fragments spill: K = 11 333 -> 543 us)
   const int sub = groups == 1 && tile == 4 ? ((ci / 16) % 3 == 0 ? 3 : (ci / 16) % 2 == 0 ? 2 : 1) : 1;
   int split = 1;
   if (workspace && base < 512) {
@@ -453,29 +587,14 @@ int winoMm(const float* v, const float* u, const float* bias, const float* res, 
   const dim3 grid(static_cast<unsigned>(co / 64), static_cast<unsigned>((tiles + 63) / 64),
                   static_cast<unsigned>(dilation * split));
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const bool occ3 = static_cast<int64_t>(grid.x) * grid.y * grid.z > 2 * 256;  // more than two per CU
+  const auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, p); };
   if (a == 4)
-    hipLaunchKernelGGL((lkd::winoMmKernel<2, 4, 1, 2, 1, UT>), grid, dim3(256), 0, s, p);
-  else if (a == 6 && occ3 && sub == 3)
-    hipLaunchKernelGGL((lkd::winoMmKernel<4, 6, 1, 3, 3, UT>), grid, dim3(256), 0, s, p);
-  else if (a == 6 && occ3 && sub == 2)
-    hipLaunchKernelGGL((lkd::winoMmKernel<4, 6, 1, 3, 2, UT>), grid, dim3(256), 0, s, p);
-  else if (a == 6 && occ3)
-    hipLaunchKernelGGL((lkd::winoMmKernel<4, 6, 1, 3, 1, UT>), grid, dim3(256), 0, s, p);
-  else if (a == 6 && sub == 3)
-    hipLaunchKernelGGL((lkd::winoMmKernel<4, 6, 1, 2, 3, UT>), grid, dim3(256), 0, s, p);
-  else if (a == 6 && sub == 2)
-    hipLaunchKernelGGL((lkd::winoMmKernel<4, 6, 1, 2, 2, UT>), grid, dim3(256), 0, s, p);
+    go(lkd::winoMmKernel<2, 4, 1, 1, UL>);
   else if (a == 6)
-    hipLaunchKernelGGL((lkd::winoMmKernel<4, 6, 1, 2, 1, UT>), grid, dim3(256), 0, s, p);
-  else if (groups == 2 && occ3)
-    hipLaunchKernelGGL((lkd::winoMmKernel<4, 7, 2, 3, 1, UT>), grid, dim3(256), 0, s, p);
-  else if (groups == 2)
-    hipLaunchKernelGGL((lkd::winoMmKernel<4, 7, 2, 2, 1, UT>), grid, dim3(256), 0, s, p);
-  else if (occ3)
-    hipLaunchKernelGGL((lkd::winoMmKernel<4, 7, 3, 3, 1, UT>), grid, dim3(256), 0, s, p);
+    sub == 3 ? go(lkd::winoMmKernel<4, 6, 1, 3, UL>) : sub == 2 ? go(lkd::winoMmKernel<4, 6, 1, 2, UL>)
+                                                                : go(lkd::winoMmKernel<4, 6, 1, 1, UL>);
   else
-    hipLaunchKernelGGL((lkd::winoMmKernel<4, 7, 3, 2, 1, UT>), grid, dim3(256), 0, s, p);
+    groups == 2 ? go(lkd::winoMmKernel<4, 7, 2, 1, UL>) : go(lkd::winoMmKernel<4, 7, 3, 1, UL>);
   if (split > 1) {
     hipLaunchKernelGGL(lkd::winoSplitReduceKernel,
                        dim3(static_cast<unsigned>(std::min<int64_t>((lo * co / 4 + 255) / 256, 8192))), dim3(256), 0,
@@ -494,16 +613,33 @@ int lk_hip_wino_mm_lc_f32(const float* v, const float* u, const float* bias, con
                           const float* tr, float* stats, int64_t v_rows, int64_t ci, int64_t co, int64_t lo,
                           int dilation, int groups, int kernel, int tile, float scale, void* workspace,
                           int64_t workspace_bytes, void* stream) {
-  return winoMm<false>(v, u, bias, res, out, tr, stats, v_rows, ci, co, lo, dilation, groups, kernel, tile, scale,
-                       workspace, workspace_bytes, stream);
+  return winoMm<0>(v, u, bias, res, out, tr, stats, v_rows, ci, co, lo, dilation, groups, kernel, tile, scale,
+                   workspace, workspace_bytes, stream);
 }
 
 int lk_hip_wino_mm_ut_lc_f32(const float* v, const float* ut, const float* bias, const float* res, float* out,
                              const float* tr, float* stats, int64_t v_rows, int64_t ci, int64_t co, int64_t lo,
                              int dilation, int groups, int kernel, int tile, float scale, void* workspace,
                              int64_t workspace_bytes, void* stream) {
-  return winoMm<true>(v, ut, bias, res, out, tr, stats, v_rows, ci, co, lo, dilation, groups, kernel, tile, scale,
-                      workspace, workspace_bytes, stream);
+  return winoMm<1>(v, ut, bias, res, out, tr, stats, v_rows, ci, co, lo, dilation, groups, kernel, tile, scale,
+                   workspace, workspace_bytes, stream);
+}
+
+int lk_hip_wino_mm_us_lc_f32(const float* v, const void* us, const float* bias, const float* res, float* out,
+                             const float* tr, float* stats, int64_t v_rows, int64_t ci, int64_t co, int64_t lo,
+                             int dilation, int groups, int kernel, int tile, float scale, void* workspace,
+                             int64_t workspace_bytes, void* stream) {
+  return winoMm<2>(v, static_cast<const float*>(us), bias, res, out, tr, stats, v_rows, ci, co, lo, dilation, groups,
+                   kernel, tile, scale, workspace, workspace_bytes, stream);
+}
+
+// Ut [A, Co / 64, N Ci 64] -> Us [A, Co / 64, N Ci 96] (bf16 parts), n = N Ci a multiple of 16, slabs = A Co / 64.
+int lk_hip_wino_split_u_f32(const float* ut, void* us, int64_t slabs, int64_t n, void* stream) {
+  if (slabs < 0 || n < 0 || n % 16 != 0) return 1;
+  if (slabs == 0 || n == 0) return 0;
+  hipLaunchKernelGGL(lkd::winoSplitUKernel, dim3(static_cast<unsigned>(std::min<int64_t>(lkh::ceilDiv(slabs * n * 8, 256), 8192))),
+                     dim3(256), 0, static_cast<hipStream_t>(stream), ut, static_cast<lkd::u32x4*>(us), slabs, n / 16);
+  return hipGetLastError() == hipSuccess ? 0 : 2;
 }
 
 int lk_hip_wino_adain_affine_lc_f32(const float* stats, const float* gb, float* af, int64_t s, int64_t c,
@@ -541,8 +677,8 @@ void runWinoTf(ExecCtx& ctx, const KernelArgs& a) {
 
 // wino_mm[_res][_stats]_lc_f32_gpu. ptrs: v, u, b, tr, x, [res], out, [stats]. ints: v(R, Ci), u(A, N Ci, Co),
 // b(Co), tr(T), x(L, Ci), [res(Lo, Co)], out(Lo, Co), [stats(d chunks, Co, 2)], dilation, groups, kernel,
-// padding, tile, [u_layout]; floats: [oscale]. u_layout 1 (this backend's addition; absent = 0, the reference's
-// layout): u is U tiled, Ut(A, Co / 64, N Ci 64) (winoMmKernel's UT layout).
+// padding, tile, [u_layout]; floats: [oscale]. u_layout (this backend's addition; absent = 0, the reference's
+// layout): 1, u is U tiled, Ut(A, Co / 64, N Ci 64); 2, U split, Us(A, Co / 64, N Ci 96) (winoMmKernel's UL layouts).
 template <bool RES, bool STATS>
 void runWinoMm(ExecCtx& ctx, const KernelArgs& a) {
   const int64_t vr = a.ints[0], ci = a.ints[1];
@@ -551,22 +687,30 @@ void runWinoMm(ExecCtx& ctx, const KernelArgs& a) {
   const int64_t co = a.ints[o + 1], lo = a.ints[o];
   const int d = static_cast<int>(a.ints[at]), groups = static_cast<int>(a.ints[at + 1]);
   const int k = static_cast<int>(a.ints[at + 2]), tile = static_cast<int>(a.ints[at + 4]);
-  const bool ut = a.numInts > static_cast<uint32_t>(at + 5) && a.ints[at + 5] == 1;
+  const int64_t ul = a.numInts > static_cast<uint32_t>(at + 5) ? a.ints[at + 5] : 0;
   LK_REQUIRE(ctx,
-             ut ? (a.ints[3] * 64 == co && a.ints[4] == groups * ci * 64)
-                : (a.ints[4] == co && a.ints[3] == groups * ci),
-             "wino_mm: u must be f32[A, N Ci, Co] (u_layout 1: f32[A, Co / 64, N Ci 64])");
+             ul == 1 || ul == 2 ? (a.ints[3] * 64 == co && a.ints[4] == groups * ci * (ul == 1 ? 64 : 96))
+                                : (a.ints[4] == co && a.ints[3] == groups * ci),
+             "wino_mm: u must be f32[A, N Ci, Co] (u_layout 1: f32[A, Co / 64, N Ci 64], 2: f32[A, Co / 64, N Ci 96])");
   const int64_t alpha = tile == 2 ? 4 : k == 3 ? 6 : 7;  // transform points of this kernel size and tile
   LK_REQUIRE(ctx, a.ints[2] == alpha, "wino_mm: u's leading dim must be the transform's point count");
   LK_REQUIRE(ctx, d >= 1 && vr % (static_cast<int64_t>(d) * alpha) == 0,
              "wino_mm: v rows must be a multiple of dilation * points");
   const int outp = RES ? 6 : 5;
   const float scale = RES && a.numFloats > 0 ? static_cast<float>(a.floats[0]) : 1.0f;
-  const auto mm = ut ? lk_hip_wino_mm_ut_lc_f32 : lk_hip_wino_mm_lc_f32;
+  const auto mm = ul == 1 ? winoMm<1> : ul == 2 ? winoMm<2> : winoMm<0>;
   if (mm(P<float>(a, 0), P<float>(a, 1), P<float>(a, 2), RES ? P<float>(a, 5) : nullptr, P<float>(a, outp),
          P<float>(a, 3), STATS ? P<float>(a, outp + 1) : nullptr, vr, ci, co, lo, d, groups, k, tile, scale,
          ctx.workspace, static_cast<int64_t>(ctx.workspaceBytes), ctx.stream))
     ctx.error = "wino_mm: invalid configuration";
+}
+
+// wino_split_u_f32_gpu. ptrs: ut, us. ints: ut(A, Co / 64, N Ci 64), us(A, Co / 64, N Ci 96).
+void runWinoSplitU(ExecCtx& ctx, const KernelArgs& a) {
+  LK_REQUIRE(ctx, a.ints[2] % 1024 == 0 && a.ints[3] == a.ints[0] && a.ints[4] == a.ints[1] &&
+             a.ints[5] * 2 == a.ints[2] * 3, "wino_split_u: ut f32[A, Co / 64, N Ci 64], us f32[A, Co / 64, N Ci 96]");
+  if (lk_hip_wino_split_u_f32(P<float>(a, 0), P<float>(a, 1), a.ints[0] * a.ints[1], a.ints[2] / 64, ctx.stream))
+    ctx.error = "wino_split_u: invalid configuration";
 }
 
 // wino_adain_affine_lc_f32_gpu. ptrs: stats, gb, af. ints: stats(S, C, 2), gb(2 Creal), af(3, C), dilation,
@@ -593,6 +737,7 @@ void registerWinogradKernels() {
   registerKernel({"wino_mm_res_lc_f32_gpu", G, runWinoMm<true, false>, 6, 1});
   registerKernel({"wino_mm_stats_lc_f32_gpu", G, runWinoMm<false, true>, 5, 2});
   registerKernel({"wino_mm_res_stats_lc_f32_gpu", G, runWinoMm<true, true>, 6, 2});
+  registerKernel({"wino_split_u_f32_gpu", G, runWinoSplitU, 1, 1});
   registerKernel({"wino_adain_affine_lc_f32_gpu", G, runWinoAffine, 2, 1});
 }
 

@@ -359,6 +359,17 @@ def current_graph() -> Graph | None:
 
 
 @contextlib.contextmanager
+def untraced():
+    """Ops inside run at once, also while a graph is traced (weights laid out once, captured as constants)."""
+    prev = current_graph()
+    _state.graph = None
+    try:
+        yield
+    finally:
+        _state.graph = prev
+
+
+@contextlib.contextmanager
 def tracing(graph: Graph):
     prev = current_graph()
     if graph.base_stream is None and torch.cuda.is_available():

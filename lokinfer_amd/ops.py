@@ -338,20 +338,30 @@ def wino_tf_lc_f32_gpu(x, tr, dilation, groups, kernel, padding, tile, affine=No
     return _launch("wino_tf_snake_lc_f32_gpu", [x, tr, affine, alpha], [s], attrs)
 
 
+def wino_split_u_f32_gpu(ut):
+    """(MI355X backend) U tiled f32[A, Co / 64, groups * Ci * 64] (winograd.wino_weights_t) -> U in three bf16 parts
+    whose sum it is, f32[A, Co / 64, groups * Ci * 96]: the wino_mm ops' u_layout = 2, laid out once per weight."""
+    _f32(ut, rank=3)
+    check(ut.shape[2] % 1024 == 0, "ut must be f32[A, Co / 64, groups * Ci * 64], Ci a multiple of 16")
+    return _launch("wino_split_u_f32_gpu", [ut], [(ut.shape[0], ut.shape[1], ut.shape[2] * 3 // 2)])
+
+
 def wino_mm_lc_f32_gpu(v, u, b, tr, x, dilation, groups, kernel, padding, tile, residual=None, out_scale=1.0,
                        stats=False, u_layout=0):
     """Per-point GEMM + AT output transform + bias [+ residual * out_scale] [+ per-128-row channel (mean, M2)],
     out [Lo, Co], stats [d * chunks, Co, 2]. Reference winograd.py:157-202. u_layout = 1 (MI355X backend): u is
-    U tiled, f32[A, Co / 64, groups * Ci * 64] (winograd.wino_weights_t), the same result."""
+    U tiled, f32[A, Co / 64, groups * Ci * 64] (winograd.wino_weights_t); 2: U split into its bf16 parts,
+    f32[A, Co / 64, groups * Ci * 96] (wino_split_u_f32_gpu); the same result."""
     _wino_attrs_ok(x, dilation, groups, kernel, padding, tile)
     _f32(v, rank=2)
     _f32(u, rank=3)
     _f32(b, tr, rank=1)
-    check(u_layout in (0, 1), "u_layout must be 0 or 1")
-    a, nci, co = (u.shape[0], u.shape[2] // 64, u.shape[1] * 64) if u_layout else u.shape
+    check(u_layout in (0, 1, 2), "u_layout must be 0, 1 or 2")
+    per = 96 if u_layout == 2 else 64  # u_layout 1, 2: floats per U row of a 64-column block
+    a, nci, co = (u.shape[0], u.shape[2] // per, u.shape[1] * 64) if u_layout else u.shape
     check(a == _wino.alpha_of(kernel, tile), "u must come from wino_weights for this kernel size")
-    check(nci == groups * x.shape[1] and (not u_layout or u.shape[2] % 64 == 0),
-          "u must be f32[A, groups * Ci, Co] (u_layout 1: [A, Co / 64, groups * Ci * 64])")
+    check(nci == groups * x.shape[1] and (not u_layout or u.shape[2] % per == 0),
+          "u must be f32[A, groups * Ci, Co] (u_layout 1, 2: [A, Co / 64, groups * Ci * 64 or 96])")
     check(co % 64 == 0, "Co must be a multiple of 64")
     check(b.shape[0] == co, "bias must be f32[Co]")
     check(tr.shape[0] == a * (a + tile), "bad transform table")
@@ -362,7 +372,7 @@ def wino_mm_lc_f32_gpu(v, u, b, tr, x, dilation, groups, kernel, padding, tile, 
         shapes.append((_wino.stats_chunks(lo, dilation) * dilation, co, 2))
     attrs = dict(dilation=int(dilation), groups=int(groups), kernel=int(kernel), padding=int(padding), tile=int(tile))
     if u_layout:
-        attrs["u_layout"] = 1
+        attrs["u_layout"] = int(u_layout)
     sfx = "_stats" if stats else ""
     if residual is None:
         check(out_scale == 1.0, "out_scale needs a residual")

@@ -249,3 +249,83 @@ def test_wino_u_layouts_agree(gpu, ci, co, l, k, d):
                                            u_layout=1)
     assert np.array_equal(y0.numpy(), y1.numpy())
     assert np.array_equal(s0.numpy(), s1.numpy())
+
+
+@pytest.mark.parametrize("ci,co,l,k,d", [(16, 64, 1, 3, 1), (32, 64, 129, 3, 1), (48, 128, 255, 3, 5), (16, 64, 300, 4, 1),
+                                         (80, 64, 515, 7, 3), (64, 128, 259, 11, 5), (1104, 1024, 300, 3, 1)])
+def test_wino_split_u(gpu, ci, co, l, k, d):
+    """u_layout 2 (U in three bf16 parts): the same MFMAs as the other layouts, so the same bits, through every chunk
+    count per step (16, 32, 48 channels), one to three tap groups, ragged tiles and the split-K path."""
+    lk = gpu
+    r, x, w, b = _case(ci + l + 5 * k, l, ci, co, k)
+    u, tr = W.wino_weights(w)
+    us = lk.ops.wino_split_u_f32_gpu(G(lk, W.wino_weights_t(w)[0]))
+    kw = dict(padding=_pad(k, d), dilation=d, stats=True)
+    y0, s0 = lk.ops.conv1d_wino_lc_f32_gpu(G(lk, x), G(lk, u), G(lk, b), G(lk, tr), k, **kw)
+    y2, s2 = lk.ops.conv1d_wino_lc_f32_gpu(G(lk, x), us, G(lk, b), G(lk, tr), k, u_layout=2, **kw)
+    assert np.array_equal(y0.numpy(), y2.numpy()) and np.array_equal(s0.numpy(), s2.numpy())
+    close(y2, _direct(x, w, b, _pad(k, d), d), 2e-4)
+
+
+def test_wino_split_u_parts(gpu):
+    """The parts sum to the value exactly, in fragment order, from denormal-free small to the largest floats."""
+    lk = gpu
+    r = np.random.default_rng(5)
+    ut = (r.standard_normal((2, 2, 2048)) * 10.0 ** r.integers(-25, 25, (2, 2, 2048))).astype(np.float32)
+    ut[0, 0, :6] = [np.inf, -np.inf, 3.4e38, -3.4028235e38, 3.39616e38, 0.0]
+    us = lk.ops.wino_split_u_f32_gpu(G(lk, ut)).numpy().view(np.uint16).reshape(2, 2, 2, 2, 3, 64, 8)
+    p = (us.astype(np.uint32) << 16).view(np.float32)
+    with np.errstate(over="ignore", invalid="ignore"):
+        back = (p[..., 0, :, :] + p[..., 1, :, :]) + p[..., 2, :, :]  # slab, cb, half, set, lane, k
+    back = back.reshape(2, 2, 2, 2, 2, 32, 2, 4).transpose(0, 1, 3, 4, 6, 2, 5, 7)  # set, k8, k4, half, col, k
+    assert np.array_equal(back.reshape(ut.shape), ut)
+
+
+def _mm_exact(v, u, tr, lo, k, a):
+    """wino_mm of d = 1 in float64 from its operands: y[t M + j] = sum_xi AT[j, xi] sum_g V[xi, t + g] U[xi, g]."""
+    n, co = W.variant(k)[1], u.shape[2]
+    v = v.astype(np.float64).reshape(a, -1, v.shape[1])
+    t = -(-lo // 4)
+    at = tr[a * a:].astype(np.float64).reshape(4, a)
+    with np.errstate(all="ignore"):
+        m = sum(v[:, g:g + t] @ u[:, g * v.shape[2]:(g + 1) * v.shape[2]].astype(np.float64) for g in range(n))
+        y = sum(at[:, x, None, None] * m[x][None] for x in range(a))
+    return y.transpose(1, 0, 2).reshape(4 * t, co)[:lo]
+
+
+@pytest.mark.parametrize("layout", [0, 2])
+@pytest.mark.parametrize("ci,l,k", [(32, 300, 3), (48, 150, 11), (1024, 70, 3)])
+def test_wino_mm_extreme_operands(gpu, ci, l, k, layout):
+    """Operands the three-part split cannot hold (infinities, NaN, values past the largest bf16) give what the f32 sum
+    gives, and rows of very different magnitude keep f32's relative error each."""
+    lk = gpu
+    r, x, w, b = _case(ci + l + k, l, ci, 64, k)
+    u, tr = W.wino_weights(w)
+    a, n = u.shape[0], W.variant(k)[1]
+    us = lk.ops.wino_split_u_f32_gpu(G(lk, W.wino_weights_t(w)[0])) if layout == 2 else G(lk, u)
+    kw = dict(dilation=1, groups=n, kernel=k, padding=_pad(k, 1), tile=4)
+    rows = W.tiles_rows(l, 1, n, 4, k)
+    scale = 10.0 ** r.integers(-15, 15, (1, rows // a, 1))
+    base = (r.standard_normal((a, rows // a, ci)) * scale).reshape(rows, ci).astype(np.float32)
+    zero = np.zeros(64, np.float32)
+
+    def run(v):
+        return lk.ops.wino_mm_lc_f32_gpu(G(lk, v), us, G(lk, zero), G(lk, tr), G(lk, x), u_layout=layout, **kw).numpy()
+
+    ref, got = _mm_exact(base, u, tr, l, k, a), run(base)
+    # each output row: n ci products per point and A points summed in f32, bounded by sqrt(n ci A) 2^-24 of the rms of
+    # its terms' magnitudes, times 16 for the largest of the row
+    at = np.abs(tr[a * a:]).reshape(4, a)
+    mag = _mm_exact(np.abs(base), np.abs(u), np.concatenate([tr[:a * a], at.ravel()]), l, k, a)
+    assert (np.abs(got - ref).max(1) <= 16 * 2.0 ** -24 * mag.max(1)).all()
+    for bad in (np.inf, -np.inf, np.nan, 3.4e38):
+        v = base / np.float32(1e15)
+        v[rows // a + 3, 5] = bad
+        v[2 * (rows // a) + 9, ci - 1] = bad
+        ref, got = _mm_exact(v, u, tr, l, k, a), run(v)
+        big = np.abs(ref) > 3e38  # overflows in f32
+        assert np.array_equal(np.isnan(ref), np.isnan(got))
+        ok = np.isfinite(ref) & ~big
+        assert np.isfinite(got[ok]).all()
+        inf = np.isinf(ref)
+        assert np.array_equal(got[inf], ref[inf].astype(np.float32))
