@@ -264,6 +264,18 @@ int lk_hip_wino_split_u_f32(const float* ut, void* us, int64_t slabs, int64_t n,
 int lk_hip_wino_adain_affine_lc_f32(const float* stats, const float* gb, float* af, int64_t s, int64_t c,
                                     int64_t creal, int dilation, int64_t length, float eps, void* stream);
 
+/* ---- f32 GEMM over split weights (MI355X backend): the weight in three exact bf16 parts, laid out once in
+ *      matrix-fragment order, the products on the bf16 matrix cores at f32 precision ---- */
+/* w f32[K, N] (nt = 0) or f32[N, K] (nt = 1) -> ws, ceil(N / 32) ceil(K / 16) 3072 bytes */
+int lk_hip_split_weight_f32(const float* w, void* ws, int64_t n, int64_t k, int nt, void* stream);
+/* out[M, N] = (act(a[M, K] W + bias) + res) * scale (act 0 none, 1 ReLU, 2 gelu_tanh; bias, res optional); K % 8 == 0,
+ * a and ws 16-byte aligned */
+int lk_hip_gemm_ws_f32(const float* a, const void* ws, const float* bias, const float* res, float* out, int64_t m,
+                       int64_t n, int64_t k, int act, float scale, void* stream);
+/* the raw sums of `planes` (1 .. 64) equal K ranges, part [planes, M, N], for lk_hip_add_bias_ln_sk_f32 */
+int lk_hip_gemm_ws_splitk_f32(const float* a, const void* ws, float* part, int64_t m, int64_t n, int64_t k, int planes,
+                              void* stream);
+
 /* ---- f16 language model (Qwen3-ASR LM; reference f16 GPU op family kernels/gpu/f16_gpu.cpp:1011-1050, contracts
  *      python/lokinfer/ops/f16.py, f16_gpu.py). f16 storage (pointers to IEEE half), f32 math and accumulation, one
  *      rounding at each output. Weights of the GEMM-like ops are packed once as W^T f16[N', K]

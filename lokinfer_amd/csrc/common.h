@@ -76,8 +76,18 @@ void registerSignalKernels();
 void registerDecodeFusedKernels();
 void registerWinogradKernels();
 void registerF16Kernels();
+void registerGemmSplitKernels();
 
 inline unsigned ceilDiv(int64_t a, int64_t b) { return static_cast<unsigned>((a + b - 1) / b); }
+
+// Split-K pays while the 64 x 64 output tiles leave most of the 256 CUs idle; above that (and for M = 1, where the
+// work is one GEMV) the producer writes one plane and the consumer reads one. The rule is shared by
+// gemm_splitk / gemm_auto_sk / gemm_ws_splitk and add_bias_layernorm2_sk (reference splitKEffective, transformer_gpu.cpp:253-268,
+// whose threshold is tuned for its own GPU).
+constexpr int64_t kSplitKMaxTiles = 64;
+inline int64_t splitKPlanes(int64_t m, int64_t n, int64_t splits) {
+  return m > 1 && ((m + 63) / 64) * ((n + 63) / 64) < kSplitKMaxTiles ? splits : 1;
+}
 
 template <typename T>
 inline T* P(const KernelArgs& a, int i) {

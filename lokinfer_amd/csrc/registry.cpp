@@ -328,15 +328,6 @@ void runAttnGen(ExecCtx& ctx, const KernelArgs& a) {
          "attention_gen: attention_cache failed");
 }
 
-// Split-K pays while the 64 x 64 output tiles leave most of the 256 CUs idle; above that (and for M = 1, where the
-// work is one GEMV) the producer writes one plane and the consumer reads one. The rule is shared by
-// gemm_splitk / gemm_auto_sk and add_bias_layernorm2_sk (reference splitKEffective, transformer_gpu.cpp:253-268,
-// whose threshold is tuned for its own GPU).
-constexpr int64_t kSplitKMaxTiles = 64;
-int64_t splitKPlanes(int64_t m, int64_t n, int64_t splits) {
-  return m > 1 && ((m + 63) / 64) * ((n + 63) / 64) < kSplitKMaxTiles ? splits : 1;
-}
-
 // gemm_splitk / gemm_auto_sk: a[M, K], b[K, N] -> out[S, M, N]; attrs splits, tile. Planes past splitKPlanes are
 // not written (their consumer does not read them).
 template <bool AUTO>
@@ -594,6 +585,7 @@ static void registerAll() {
     registerDecodeFusedKernels();
     registerWinogradKernels();
     registerF16Kernels();
+    registerGemmSplitKernels();
     std::sort(names().begin(), names().end());
   });
 }

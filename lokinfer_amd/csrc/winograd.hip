@@ -129,19 +129,6 @@ struct WinoMmArgs {
   float scale;
 };
 
-// The three bf16 parts of 8 values, in r[0 .. 2], become the values themselves, in r[0] and r[1].
-__device__ __forceinline__ void joinParts(f32x4 (&r)[3]) {
-  const u32x4 h = __builtin_bit_cast(u32x4, r[0]), m = __builtin_bit_cast(u32x4, r[1]);
-  const u32x4 l = __builtin_bit_cast(u32x4, r[2]);
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int o = 0; o < 2; ++o) {
-      const auto f = [&](unsigned x) { return __uint_as_float(o ? x & 0xffff0000u : x << 16); };
-      r[i >> 1][2 * (i & 1) + o] = (f(h[i]) + f(m[i])) + f(l[i]);
-    }
-}
-
 // MFMA-bound: the products run on the bf16 matrix cores as three-part splits (split3.h), 6 N S MFMAs of 32 cycles per
 // wave and step of S 16-channel chunks, at three workgroups per CU (at most 168 registers): the y accumulators leave
 // room for one 32 x 32 block per wave, and it takes three waves per SIMD to cover a step's loads, LDS stores and
@@ -464,8 +451,7 @@ __global__ __launch_bounds__(256, 3) void winoMmKernel(WinoMmArgs p) {
   }
 }
 
-// Ut (u_layout 1) -> Us (u_layout 2), a fragment's 8 values per thread. Parts of a value that would round past the
-// largest bf16 are cut instead of rounded, infinities and NaN are h alone, so that the parts always sum to the value.
+// Ut (u_layout 1) -> Us (u_layout 2), a fragment's 8 values per thread.
 __global__ __launch_bounds__(256) void winoSplitUKernel(const float* __restrict__ ut, u32x4* __restrict__ us,
                                                        int64_t slabs, int64_t sets) {
   const int64_t total = slabs * sets * 128;
@@ -474,19 +460,11 @@ __global__ __launch_bounds__(256) void winoSplitUKernel(const float* __restrict_
     const int lane = static_cast<int>(i & 63), half = static_cast<int>(i >> 6) & 1;
     const int64_t set = (i >> 7) % sets, slab = (i >> 7) / sets;
     const float* src = ut + (slab * sets + set) * 1024 + ((lane >> 5) * 128 + half * 32 + (lane & 31)) * 4;
+    float v[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) v[k] = src[(k >> 2) * 256 + (k & 3)];
     u32x4 parts[3];
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      float rest = src[(k >> 2) * 256 + (k & 3)];
-      const bool finite = fabsf(rest) <= 3.40282347e38f, cut = fabsf(rest) >= 3.38953139e38f;
-#pragma unroll
-      for (int q = 0; q < 3; ++q) {
-        const unsigned b = __float_as_uint(rest);
-        const unsigned part = (cut || !finite ? b : b + 0x7fff + ((b >> 16) & 1)) >> 16;
-        rest = finite ? rest - __uint_as_float(part << 16) : 0.0f;
-        parts[q][k >> 1] = k & 1 ? parts[q][k >> 1] | part << 16 : part;
-      }
-    }
+    splitExact(v, parts);
 #pragma unroll
     for (int q = 0; q < 3; ++q) us[((slab * 2 + half) * sets + set) * 192 + q * 64 + lane] = parts[q];
   }

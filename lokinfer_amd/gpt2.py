@@ -13,8 +13,8 @@ so a step is one captured HIP graph.
 
 Gpt2Generator is the reference's `build_generate` (models/gpt2.py:250-333): chunked prefill and decode over the same
 persistent caches. A call with T new tokens at start position pos returns the logits of the last one; T = 1 runs the
-decode step above, T > 1 the chunk forward (GEMM, kv_write_rows + flash attention over the cache, split-K
-projections into bias + residual + LayerNorm).
+decode step above, T > 1 the chunk forward (GEMMs over split weights, kv_write_rows + flash attention over the
+cache, split-K projections into bias + residual + LayerNorm).
 
 By default (fused=True) each layer runs the same arithmetic in 5 launches instead of 13: the GEMVs write
 row-slice partial sums and the consumer of each GEMV sums the slices itself (the decode-attention chunk kernel
@@ -139,7 +139,7 @@ class Gpt2Decoder:
 
 class Gpt2Generator(Gpt2Decoder):
     """Chunked prefill + decode sharing the caches (reference build_generate, models/gpt2.py:250-333). sk: split-K
-    factors of the two N = 768 projections for T > 1 ((0, 0) = plain GEMM + add_bias_layernorm2). chunk_graph:
+    factors of the two N = 768 projections for T > 1 ((0, 0) = one sum + add_bias_layernorm2). chunk_graph:
     capture each chunk length's forward as a HIP graph (pays off when one length recurs; a one-off prompt runs
     eagerly)."""
 
@@ -149,6 +149,9 @@ class Gpt2Generator(Gpt2Decoder):
         self.sk = tuple(sk)
         dev = self.w["transformer.wte.weight"].t.device
         self.positions = torch.arange(N_POS, dtype=torch.int64, device=dev)  # device pos views, no host copies
+        # the chunk forward's projections run over split weights (the decode step streams the plain ones)
+        self.ws = {k: ops.split_weight(v) for k, v in self.w.items()
+                   if k.endswith(("attn.c_attn.weight", "attn.c_proj.weight", "mlp.c_fc.weight", "mlp.c_proj.weight"))}
         self.chunk_model = lk_capture(self._chunk, graph=chunk_graph)
 
     def _chunk(self, ids: Tensor, pos: Tensor):
@@ -160,20 +163,20 @@ class Gpt2Generator(Gpt2Decoder):
         ln = ops.layernorm_f32_gpu(h, w[P + "h.0.ln_1.weight"], w[P + "h.0.ln_1.bias"], eps=LN_EPS)
 
         def proj_ln(x, wk, res, ln_key, splits):  # (res + x @ W + b, LN of it)
-            if splits:
-                parts = ops.gemm_auto_sk_f32_gpu(x, w[wk + "weight"], splits)
+            if splits and ops.splitk_planes(T, D, splits) > 1:
+                parts = ops.gemm_ws_splitk_f32_gpu(x, self.ws[wk + "weight"], splits)
                 return ops.add_bias_layernorm2_sk_f32_gpu(parts, w[wk + "bias"], res, w[ln_key + "weight"],
                                                           w[ln_key + "bias"], eps=LN_EPS)
-            return ops.add_bias_layernorm2_f32_gpu(ops.gemm_auto_f32_gpu(x, w[wk + "weight"]), w[wk + "bias"], res,
+            return ops.add_bias_layernorm2_f32_gpu(ops.gemm_ws_f32_gpu(x, self.ws[wk + "weight"]), w[wk + "bias"], res,
                                                    w[ln_key + "weight"], w[ln_key + "bias"], eps=LN_EPS)
 
         for i, (kc, vc) in enumerate(self.caches):
             L = f"{P}h.{i}."
             nxt = f"{P}h.{i + 1}.ln_1." if i + 1 < N_LAYER else P + "ln_f."
-            qkv = ops.gemm_auto_f32_gpu(ln, w[L + "attn.c_attn.weight"])
+            qkv = ops.gemm_ws_f32_gpu(ln, self.ws[L + "attn.c_attn.weight"])
             att = ops.attention_gen2_f32_gpu(qkv, kc, vc, pos, w[L + "attn.c_attn.bias"], heads=HEADS)
             h, ln = proj_ln(att, L + "attn.c_proj.", h, L + "ln_2.", self.sk[0])
-            f = ops.gemm_auto_bias_gelu_f32_gpu(ln, w[L + "mlp.c_fc.weight"], w[L + "mlp.c_fc.bias"])
+            f = ops.gemm_ws_f32_gpu(ln, self.ws[L + "mlp.c_fc.weight"], w[L + "mlp.c_fc.bias"], act="gelu")
             h, ln = proj_ln(f, L + "mlp.c_proj.", h, nxt, self.sk[1])
         logits = ops.gemm_nt_f32_gpu_mps(ops.view(ln, [1, D], offset=(T - 1) * D), w[P + "wte.weight"])
         return logits, ops.argmax_f32_gpu(logits)

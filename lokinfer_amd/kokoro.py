@@ -112,6 +112,15 @@ class KokoroGpu:
             self._g[key] = t
         return t
 
+    def split_w(self, key: str, make) -> "ops.SplitWeight":
+        """The torch linear weight [out, in] of `make` as the split-weight GEMM's operand, laid out once."""
+        k = key + "#split"
+        if k not in self._g:
+            with untraced():
+                self._g[k] = ops.split_weight(from_numpy(np.ascontiguousarray(make(), np.float32), device="gpu", copy=True),
+                                              nt=True)
+        return self._g[k]
+
     def _bank(self, root: str):
         """All `<root>.*.fc` style projections as one [128, total] weight (one GEMV per style vector), with each
         fc's (offset, width) (reference W.style_bank, model.py:67-81)."""
@@ -262,31 +271,32 @@ class KokoroGpu:
         M = "bert.encoder.embedding_hidden_mapping_in"
         h = ops.gemm_bias_f32_gpu(e, self.g(M + ".weight", _t), self.g(M + ".bias"))
         L = "bert.encoder.albert_layer_groups.0.albert_layers.0."
-        # the plain projections run as NT GEMMs on the [out, in] weights (the GEMM's B fragments are then 16-byte
-        # runs of K); the result is the reference's x . W^T
-        wqkv = self.const("albert#wqkv_nt", lambda: np.concatenate(
+        wqkv = self.split_w("albert#wqkv", lambda: np.concatenate(
             [self.sd[L + f"attention.{n}.weight"] for n in ("query", "key", "value")], axis=0))
         bqkv = self.const("albert#bqkv", lambda: np.concatenate(
             [self.sd[L + f"attention.{n}.bias"] for n in ("query", "key", "value")]))
-        # Below 64 output tiles (T <= 320) the projections feeding a LayerNorm split K over workgroups; their
-        # partial planes then go straight into the LayerNorm, which sums them (add_bias_layernorm2_sk), instead of
-        # through a reduction launch of their own (59 tokens: 24 launches fewer)
-        sk = ops.splitk_planes(t, 768, 3) > 1
 
-        def proj_ln(x, w, splits, b, g, beta):
-            if sk:
-                parts = ops.gemm_splitk_f32_gpu(x, self.g(w, _t), splits)
-                return ops.add_bias_layernorm2_sk_f32_gpu(parts, self.g(b), h, self.g(g), self.g(beta), eps=1e-12)[1]
-            return ops.add_bias_layernorm_f32_gpu(ops.gemm_nt_f32_gpu_mps(x, self.g(w)), self.g(b), h, self.g(g),
-                                                  self.g(beta), eps=1e-12)
+        # Below 64 output tiles (T <= 320) the FFN's 2048-deep output projection splits K over workgroups too, its planes
+        # summed by the LayerNorm
+        sk = ops.splitk_planes(t, 768, 4) > 1
+
+        def linear(x, p, **kw):
+            return ops.gemm_ws_f32_gpu(x, self.split_w(L + p, lambda: self.sd[L + p + ".weight"]), **kw)
 
         for _ in range(12):
-            a = ops.attention_qkv_sg_f32_gpu(ops.gemm_nt_f32_gpu_mps(h, wqkv), bqkv, heads=12)
-            h = proj_ln(a, L + "attention.dense.weight", 3, L + "attention.dense.bias",
-                        L + "attention.LayerNorm.weight", L + "attention.LayerNorm.bias")
-            f = ops.gemm_steel_f32_gpu(h, self.g(L + "ffn.weight", _t), self.g(L + "ffn.bias"), act="gelu")
-            h = proj_ln(f, L + "ffn_output.weight", 8, L + "ffn_output.bias", L + "full_layer_layer_norm.weight",
-                        L + "full_layer_layer_norm.bias")
+            a = ops.attention_qkv_sg_f32_gpu(ops.gemm_ws_f32_gpu(h, wqkv), bqkv, heads=12)
+            h = ops.add_bias_layernorm_f32_gpu(linear(a, "attention.dense"), self.g(L + "attention.dense.bias"), h,
+                                               self.g(L + "attention.LayerNorm.weight"),
+                                               self.g(L + "attention.LayerNorm.bias"), eps=1e-12)
+            f = linear(h, "ffn", bias=self.g(L + "ffn.bias"), act="gelu")
+            ln = (self.g(L + "ffn_output.bias"), h, self.g(L + "full_layer_layer_norm.weight"),
+                  self.g(L + "full_layer_layer_norm.bias"))
+            if sk:
+                parts = ops.gemm_ws_splitk_f32_gpu(f, self.split_w(L + "ffn_output", lambda: self.sd[L + "ffn_output.weight"]),
+                                                   4)
+                h = ops.add_bias_layernorm2_sk_f32_gpu(parts, *ln, eps=1e-12)[1]
+            else:
+                h = ops.add_bias_layernorm_f32_gpu(linear(f, "ffn_output"), *ln, eps=1e-12)
         return h
 
     def text_encoder_cnn(self, ids: Tensor) -> Tensor:
@@ -389,7 +399,7 @@ class KokoroGpu:
         # generator
         for i, (k_up, u) in enumerate(((20, 10), (12, 6))):
             x = ops.leaky_lc_f32_gpu(x, 0.1)
-            y = ops.gemm_nt_f32_gpu_mps(x, self.g(G + f"ups.{i}.weight", _w_convt_nt))  # [Lin, K * Co]
+            y = ops.gemm_ws_f32_gpu(x, self.split_w(G + f"ups.{i}", lambda: _w_convt_nt(self.sd[G + f"ups.{i}.weight"])))
             ctx.join(self.streams[2 + i])
             x = ops.convt_gather_lc_f32_gpu(y, self.g(G + f"ups.{i}.bias"), k_up, u, (k_up - u) // 2,
                                             add=xs_stage[i], reflect_left=(i == 1))

@@ -239,6 +239,50 @@ def gemv1_bias_f32_gpu(x, w, b):
     return _launch("gemv1_bias_f32_gpu", [x, w, b], [(x.shape[0], 1)])
 
 
+# ---- GEMM over split weights (MI355X backend) ----------------------------------------------------------------
+
+class SplitWeight:
+    """A weight w f32[K, N] as three exact bf16 parts in matrix-fragment order on the device (`split_weight`); `shape`
+    is the logical (K, N)."""
+
+    def __init__(self, ws, shape):
+        self.ws, self.shape = ws, tuple(shape)
+
+
+def split_weight(w, nt: bool = False) -> SplitWeight:
+    """(MI355X backend) w f32[K, N] (nt: f32[N, K]) -> SplitWeight, laid out once for the gemm_ws ops."""
+    _f32(w, rank=2)
+    k, n = (w.shape[1], w.shape[0]) if nt else w.shape
+    return SplitWeight(_launch("split_weight_f32_gpu", [w], [(-(-n // 32), -(-k // 16) * 768)], dict(nt=int(nt))), (k, n))
+
+
+def gemm_ws_f32_gpu(a, w: SplitWeight, bias=None, act="none", residual=None):
+    """(MI355X backend) act(a f32[M, K] @ w + bias) [+ residual] with f32 precision on the bf16 matrix cores, as
+    gemm_steel_f32_gpu over a plain weight; K % 8 == 0."""
+    _f32(a, rank=2)
+    check(a.shape[1] == w.shape[0], f"gemm_ws: inner dims differ: {a.shape}, {w.shape}")
+    check(a.shape[1] % 8 == 0, "K must be a multiple of 8")
+    s = (a.shape[0], w.shape[1])
+    if bias is None:
+        check(act == "none" and residual is None, "act / residual need a bias")
+        return _launch("gemm_ws_f32_gpu", [a, w.ws], [s])
+    _bias_ok(bias, s[1])
+    if residual is not None:
+        check(act == "none" and tuple(residual.shape) == s, "residual must be f32[M, N], act none")
+        return _launch("gemm_ws_bias_res_f32_gpu", [a, w.ws, bias, residual], [s])
+    name = {"none": "gemm_ws_bias_f32_gpu", "gelu": "gemm_ws_bias_gelu_f32_gpu", "relu": "gemm_ws_bias_relu_f32_gpu"}[act]
+    return _launch(name, [a, w.ws, bias], [s])
+
+
+def gemm_ws_splitk_f32_gpu(a, w: SplitWeight, splits):
+    """(MI355X backend) gemm_splitk_f32_gpu over a split weight: partials f32[S, M, N] (rule splitk_planes) for
+    add_bias_layernorm2_sk_f32_gpu. For few rows and a long K, whose one-launch sum leaves CUs idle."""
+    _f32(a, rank=2)
+    check(a.shape[1] == w.shape[0] and a.shape[1] % 8 == 0, f"gemm_ws: a f32[M, K], K % 8 == 0: {a.shape}, {w.shape}")
+    check(1 <= int(splits) <= 64, "splits must be 1 .. 64")
+    return _launch("gemm_ws_splitk_f32_gpu", [a, w.ws], [(int(splits), a.shape[0], w.shape[1])], dict(splits=int(splits)))
+
+
 # ---- conv1d (channel-last) ----------------------------------------------------------------------------------
 
 def _conv_lc_shape(x, w, b, padding, dilation, stride):

@@ -1,0 +1,93 @@
+"""The GEMM over split weights (csrc/gemm_split.hip, ops.split_weight / gemm_ws_f32_gpu) against float64."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def lk():
+    import lokinfer_amd
+
+    return lokinfer_amd
+
+
+def G(lk, a):
+    return lk.from_numpy(np.ascontiguousarray(a, np.float32), device="gpu", copy=True)
+
+
+# (M, K, N): one kernel of the launcher's rule each (64 x 128 tiles, 32 x 128, 32 x 64 with K over two / four wave groups,
+# 32 x 32 over eight), with ragged rows, columns and K tails, K shorter than the wave groups, single rows and columns
+SHAPES = [(1, 8, 1), (1, 16, 33), (31, 24, 32), (33, 40, 31), (59, 768, 2304), (200, 2048, 96), (487, 768, 768),
+          (500, 72, 700), (487, 2056, 770), (1030, 136, 2100), (4100, 40, 2090), (8200, 256, 1056)]
+
+
+@pytest.mark.parametrize("m,k,n", SHAPES)
+def test_gemm_ws(lk, m, k, n):
+    r = np.random.default_rng(m + 3 * k + 7 * n)
+    a, w = r.standard_normal((m, k)).astype(np.float32), r.standard_normal((k, n)).astype(np.float32)
+    ref, mag = a.astype(np.float64) @ w, np.abs(a).astype(np.float64) @ np.abs(w)
+    bound = 2.0 ** -24 * (4 + np.sqrt(k)) * mag  # f32 sums of k products; random signs leave far less
+    nn, nt = lk.ops.split_weight(G(lk, w)), lk.ops.split_weight(G(lk, w.T), nt=True)
+    assert nn.shape == nt.shape == (k, n) and np.array_equal(nn.ws.numpy().view(np.uint8), nt.ws.numpy().view(np.uint8))
+    y = lk.ops.gemm_ws_f32_gpu(G(lk, a), nn).numpy()
+    assert y.shape == (m, n) and (np.abs(y - ref) <= bound).all()
+    b, res = r.standard_normal(n).astype(np.float32), r.standard_normal((m, n)).astype(np.float32)
+    z = lk.ops.gemm_ws_f32_gpu(G(lk, a), nn, G(lk, b), act="relu").numpy()
+    assert (np.abs(z - np.maximum(ref + b, 0)) <= bound + 2.0 ** -23 * np.abs(ref + b)).all()
+    z = lk.ops.gemm_ws_f32_gpu(G(lk, a), nn, G(lk, b), residual=G(lk, res)).numpy()
+    assert (np.abs(z - (ref + b + res)) <= bound + 2.0 ** -22 * (np.abs(ref) + np.abs(b) + np.abs(res))).all()
+    x = ref + b
+    gelu = 0.5 * x * (1 + np.tanh(np.sqrt(2 / np.pi) * (x + 0.044715 * x ** 3)))
+    z = lk.ops.gemm_ws_f32_gpu(G(lk, a), nn, G(lk, b), act="gelu").numpy()
+    assert (np.abs(z - gelu) <= 1.2 * bound + 1e-6 * (1 + np.abs(x))).all()  # |gelu'| <= 1.13; f32 tanh
+
+
+@pytest.mark.parametrize("m,k,n", [(33, 40, 70), (200, 768, 64), (487, 768, 768), (8200, 64, 1056)])
+def test_gemm_ws_extreme_operands(lk, m, k, n):
+    """Infinities, NaN and values past the largest bf16 give what the f32 sum gives; rows of very different magnitude
+    keep f32's relative error each; a weight holding such values too."""
+    r = np.random.default_rng(m + k + n)
+    a = (r.standard_normal((m, k)) * 10.0 ** r.integers(-18, 18, (m, 1))).astype(np.float32)
+    w = r.standard_normal((k, n)).astype(np.float32)
+    y = lk.ops.gemm_ws_f32_gpu(G(lk, a), lk.ops.split_weight(G(lk, w))).numpy()
+    assert (np.abs(y - a.astype(np.float64) @ w) <= 2.0 ** -24 * (4 + np.sqrt(k)) * (np.abs(a).astype(np.float64) @ np.abs(w))).all()
+    a = r.standard_normal((m, k)).astype(np.float32)
+    for where in ("a", "w"):
+        for bad in (np.inf, -np.inf, np.nan, 3.4e38):
+            x, v = a.copy(), w.copy()
+            if where == "a":
+                x[m // 2, 3] = bad
+            else:
+                v[5, n - 1] = bad
+                v[k - 1, 0] = bad
+            with np.errstate(all="ignore"):
+                ref = x.astype(np.float64) @ v
+                bound = 2.0 ** -24 * (4 + np.sqrt(k)) * (np.abs(x).astype(np.float64) @ np.abs(v))  # f32 sums of k products
+            got = lk.ops.gemm_ws_f32_gpu(G(lk, x), lk.ops.split_weight(G(lk, v))).numpy()
+            with np.errstate(all="ignore"):
+                fits = np.abs(ref) < 3e38
+                assert np.array_equal(np.isnan(ref), np.isnan(got))
+                assert np.array_equal(got[np.isinf(ref)], ref[np.isinf(ref)].astype(np.float32))
+                assert (np.abs(got[fits] - ref[fits]) <= bound[fits]).all()
+
+
+@pytest.mark.parametrize("m,k,n,s", [(1, 64, 40, 3), (2, 16, 31, 5), (59, 2048, 768, 4), (320, 136, 700, 7), (400, 256, 768, 4)])
+def test_gemm_ws_splitk(lk, m, k, n, s):
+    r = np.random.default_rng(m + k)
+    a, w = r.standard_normal((m, k)).astype(np.float32), r.standard_normal((k, n)).astype(np.float32)
+    parts = lk.ops.gemm_ws_splitk_f32_gpu(G(lk, a), lk.ops.split_weight(G(lk, w)), s).numpy()
+    assert parts.shape == (s, m, n)
+    y = parts[:lk.ops.splitk_planes(m, n, s)].astype(np.float64).sum(0)
+    bound = 2.0 ** -24 * (4 + np.sqrt(k)) * (np.abs(a).astype(np.float64) @ np.abs(w))  # f32 sums of k products
+    assert (np.abs(y - a.astype(np.float64) @ w) <= bound).all()
+
+
+def test_gemm_ws_refuses(lk):
+    w = lk.ops.split_weight(G(lk, np.ones((12, 4))))
+    with pytest.raises(ValueError):
+        lk.ops.gemm_ws_f32_gpu(G(lk, np.ones((2, 12))), w)  # K % 8 != 0
+    w = lk.ops.split_weight(G(lk, np.ones((16, 4))))
+    with pytest.raises(ValueError):
+        lk.ops.gemm_ws_f32_gpu(G(lk, np.ones((2, 8))), w)
+    assert lk.ops.gemm_ws_f32_gpu(G(lk, np.ones((0, 16))), w).shape == (0, 4)
