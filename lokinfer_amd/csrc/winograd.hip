@@ -33,16 +33,15 @@ typedef float v4w __attribute__((ext_vector_type(4)));
 
 constexpr int kWinoRows = 128;  // output rows per statistics chunk
 
-// V[rho, xi, r, c4 .. c4 + 3] for R = 4 consecutive tile rows r per thread, i.e. per (rho, r / R, c4), channel
-// quad fastest: the R tiles share their overlapping input rows, so a thread loads and activates M R + A - M rows
-// once (1.19x the input instead of A / M = 1.75x at M = 4, A = 7) and writes R A rows of V. act: 0 none,
-// 1 snake(affine), 2 leaky(affine); rows outside the residue class are zero (the conv pads after the activation).
-template <int M, int A>
+// V[rho, xi, r, c4 .. c4 + 3] for R consecutive tile rows r per thread, i.e. per (rho, r / R, c4), channel quad fastest:
+// the R tiles share their overlapping input rows, so a thread loads and activates M R + A - M rows once (R = 2: 1.4x
+// the input instead of A / M = 1.75x at M = 4, A = 7) and writes R A rows of V. act: 0 none, 1 snake(affine), 2
+// leaky(affine); rows outside the residue class are zero (the conv pads after the activation).
+template <int M, int A, int R>
 __global__ __launch_bounds__(256) void winoTfKernel(const float* __restrict__ x, const float* __restrict__ tr,
                                                    const float* __restrict__ af, const float* __restrict__ alpha,
                                                    float* __restrict__ v, int64_t l, int64_t c, int d, int padq,
                                                    int64_t rmax, int act, float slope) {
-  constexpr int R = 4;
   constexpr int XR = M * R + A - M;  // input rows behind R tiles
   const int64_t c4n = c / 4;
   const int64_t groups = (rmax + R - 1) / R;
@@ -510,20 +509,25 @@ int lk_hip_wino_tf_lc_f32(const float* x, const float* tr, const float* affine, 
   const int a = tile == 2 ? 4 : kernel == 3 ? 6 : 7;
   if (v_rows % (static_cast<int64_t>(dilation) * a) != 0) return 1;
   const int64_t rmax = v_rows / (static_cast<int64_t>(dilation) * a);
-  const int64_t total = static_cast<int64_t>(dilation) * ((rmax + 3) / 4) * (c / 4);  // 4 tile rows per thread
-  if (total == 0) return 0;
-  const unsigned blocks = static_cast<unsigned>(std::min<int64_t>((total + 255) / 256, 65536));
   hipStream_t s = static_cast<hipStream_t>(stream);
   const int padq = padding / dilation;
+  const auto threads = [&](int r) { return static_cast<int64_t>(dilation) * ((rmax + r - 1) / r) * (c / 4); };
+  if (threads(1) == 0) return 0;
+  const auto go = [&](auto kernel, int r) {
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(std::min<int64_t>((threads(r) + 255) / 256, 65536))),
+                       dim3(256), 0, s, x, tr, affine, alpha, v, l, c, dilation, padq, rmax, act, slope);
+  };
+  // One tile row per thread while that is what fills the chip (latency-bound: a thread's loads and stores are one round
+  // trip each), two beyond: in us with one / two / four rows per thread, (L, C, K, d) = (287, 1104, 3, 1) 4.9 / 6.2 /
+  // 8.4, (5740, 256, 7, 3) 7.5 / 8.0 / 10.2, (34441, 128, 7, 3) 13.1 / 14.3 / 15.1, (100000, 128, 11, 1) 28.7 / 28.0 /
+  // 30.2, (293281, 128, 11, 5) 86.9 / 85.1 / 89.2.
+  const auto pick = [&](auto one, auto two) { threads(1) < 524288 ? go(one, 1) : go(two, 2); };
   if (a == 4)
-    hipLaunchKernelGGL((lkd::winoTfKernel<2, 4>), dim3(blocks), dim3(256), 0, s, x, tr, affine, alpha, v, l, c,
-                       dilation, padq, rmax, act, slope);
+    pick(lkd::winoTfKernel<2, 4, 1>, lkd::winoTfKernel<2, 4, 2>);
   else if (a == 6)
-    hipLaunchKernelGGL((lkd::winoTfKernel<4, 6>), dim3(blocks), dim3(256), 0, s, x, tr, affine, alpha, v, l, c,
-                       dilation, padq, rmax, act, slope);
+    pick(lkd::winoTfKernel<4, 6, 1>, lkd::winoTfKernel<4, 6, 2>);
   else
-    hipLaunchKernelGGL((lkd::winoTfKernel<4, 7>), dim3(blocks), dim3(256), 0, s, x, tr, affine, alpha, v, l, c,
-                       dilation, padq, rmax, act, slope);
+    pick(lkd::winoTfKernel<4, 7, 1>, lkd::winoTfKernel<4, 7, 2>);
   return hipGetLastError() == hipSuccess ? 0 : 2;
 }
 
