@@ -23,13 +23,15 @@ namespace lkd {
 
 constexpr int kStatChunk = 128;
 
-// Block = 64 channels x 4 row groups of one 128-row chunk. Pass 1: mean; pass 2: centred M2 (the chunk's rows are
-// re-read from L2). Dilation d: the chunks of each residue class rho (rows rho + d i, i < ceil((L - rho) / d)), block
+// Block = 64 channels x G groups of 128 / G rows of one 128-row chunk. Pass 1: mean; pass 2: centred M2, both from the
+// rows held in registers. Dilation d: the chunks of each residue class rho (rows rho + d i, i < ceil((L - rho) / d)), block
 // y = rho chunks + k over rows rho + d (128 k + i), written to st[(rho chunks + k) C + c] (the Winograd GEMM's
 // statistics layout; d = 1 is the plain 128-row layout). Chunks past a residue class's rows write nothing.
-__global__ __launch_bounds__(256) void statsKernel(const float* __restrict__ x, float* __restrict__ st, int64_t l,
-                                                  int64_t c, int d, int64_t chunks) {
-  __shared__ float part[4][64];
+template <int G>
+__global__ __launch_bounds__(64 * G) void statsKernel(const float* __restrict__ x, float* __restrict__ st, int64_t l,
+                                                     int64_t c, int d, int64_t chunks) {
+  constexpr int ROWS = kStatChunk / G;  // rows per thread
+  __shared__ float part[G][64];
   const int cl = threadIdx.x & 63, g = threadIdx.x >> 6;
   const int64_t ch = static_cast<int64_t>(blockIdx.x) * 64 + cl;
   const int64_t s = blockIdx.y;
@@ -39,23 +41,29 @@ __global__ __launch_bounds__(256) void statsKernel(const float* __restrict__ x, 
   const int n = static_cast<int>(min<int64_t>(kStatChunk, lor - t0));
   if (n <= 0) return;  // uniform over the block
   const bool ok = ch < c;
-  const int r0 = g * 32;
+  const int r0 = g * ROWS;
   const int64_t stride = static_cast<int64_t>(d) * c;
   const float* col = x + (rho + t0 * d) * c + (ok ? ch : 0);
-  // the thread's 32 rows are loaded once (independent loads in flight) and kept for both passes
-  float v[32];
+  // the thread's rows are loaded once (independent loads in flight) and kept for both passes
+  float v[ROWS];
 #pragma unroll
-  for (int i = 0; i < 32; ++i) v[i] = (ok && r0 + i < n) ? col[static_cast<int64_t>(r0 + i) * stride] : 0.0f;
+  for (int i = 0; i < ROWS; ++i) v[i] = (ok && r0 + i < n) ? col[static_cast<int64_t>(r0 + i) * stride] : 0.0f;
   float sum = 0.0f;
 #pragma unroll
-  for (int i = 0; i < 32; ++i) sum += v[i];
+  for (int i = 0; i < ROWS; ++i) sum += v[i];
   part[g][cl] = sum;
   __syncthreads();
-  const float mean = (part[0][cl] + part[1][cl] + part[2][cl] + part[3][cl]) / static_cast<float>(n);
+  auto total = [&] {
+    float t = part[0][cl];
+#pragma unroll
+    for (int i = 1; i < G; ++i) t += part[i][cl];
+    return t;
+  };
+  const float mean = total() / static_cast<float>(n);
   __syncthreads();
   float m2 = 0.0f;
 #pragma unroll
-  for (int i = 0; i < 32; ++i) {
+  for (int i = 0; i < ROWS; ++i) {
     const float dv = v[i] - mean;
     if (r0 + i < n) m2 += dv * dv;
   }
@@ -63,7 +71,7 @@ __global__ __launch_bounds__(256) void statsKernel(const float* __restrict__ x, 
   __syncthreads();
   if (g == 0 && ok) {
     st[(s * c + ch) * 2] = mean;
-    st[(s * c + ch) * 2 + 1] = part[0][cl] + part[1][cl] + part[2][cl] + part[3][cl];
+    st[(s * c + ch) * 2 + 1] = total();
   }
 }
 
@@ -360,7 +368,12 @@ namespace lkh {
 int residueStats(const float* x, float* st, int64_t l, int64_t c, int d, int64_t chunks, hipStream_t s) {
   if (l <= 0 || c <= 0 || d < 1 || chunks < 1) return 1;
   dim3 grid(static_cast<unsigned>(ceilDiv(c, 64)), static_cast<unsigned>(d * chunks));
-  hipLaunchKernelGGL(lkd::statsKernel, grid, dim3(256), 0, s, x, st, l, c, d, chunks);
+  // short loads per thread while a block's latency is what the launch takes, long ones where it streams: G = 4 / 8 at
+  // 287 x 1024 4.8 / 3.8 us, 5740 x 256 4.9 / 3.9, 34441 x 128 5.4 / 5.2, 293281 x 128 26.4 / 28.1
+  if (static_cast<int64_t>(grid.x) * grid.y < 2048)
+    hipLaunchKernelGGL(lkd::statsKernel<8>, grid, dim3(512), 0, s, x, st, l, c, d, chunks);
+  else
+    hipLaunchKernelGGL(lkd::statsKernel<4>, grid, dim3(256), 0, s, x, st, l, c, d, chunks);
   return hipGetLastError() == hipSuccess ? 0 : 2;
 }
 }  // namespace lkh
@@ -371,10 +384,7 @@ extern "C" {
 
 int lk_hip_channel_stats_lc_f32(const float* x, float* st, int64_t l, int64_t c, void* stream) {
   if (l <= 0 || c <= 0) return 1;
-  const int64_t chunks = lkh::ceilDiv(l, lkd::kStatChunk);
-  dim3 grid(lkh::ceilDiv(c, 64), chunks);
-  hipLaunchKernelGGL(lkd::statsKernel, grid, dim3(256), 0, static_cast<hipStream_t>(stream), x, st, l, c, 1, chunks);
-  LK_RET;
+  return lkh::residueStats(x, st, l, c, 1, lkh::ceilDiv(l, lkd::kStatChunk), static_cast<hipStream_t>(stream));
 }
 
 int lk_hip_adain_affine_lc_f32(const float* st, const float* gb, float* af, int64_t l, int64_t c, int64_t creal,
