@@ -182,8 +182,7 @@ class KokoroGpu:
         af2 = self.affine(h, bank, p + ".norm2.fc", hst, hd)
         sc = ops.upsample2_lc_f32_gpu(x) if upsample else x
         if p + ".conv1x1.weight" in self.sd:
-            sc = ops.conv1d_lc_f32_gpu(sc, self.g(p + ".conv1x1.weight", _w_lc),
-                                       self.const(f"zeros#{cout}", lambda: np.zeros(cout)))
+            sc = ops.gemm_ws_f32_gpu(sc, self.split_w(p + ".conv1x1", lambda: _w_lc(self.sd[p + ".conv1x1.weight"])[:, 0]))
         return self.conv(h, p + ".conv2", af2, 3, act="leaky", slope=0.2, residual=sc, out_scale=SQRT1_2)[0]
 
     def wino(self, key: str, ci_pad: int, co_pad: int):
