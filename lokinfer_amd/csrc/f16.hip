@@ -666,16 +666,26 @@ __global__ __launch_bounds__(256) void gemmF16ReduceKernel(GemmF16Params p) {
 }
 
 // ---- causal GQA over the caches, T > 1: flash tiles on MFMA --------------------------------------------------
-// Workgroup = NW waves = 32 queries (positions pos + q0 ..) of one q head; wave w takes key tiles w, w + NW, ...
-// (32 keys each) of the head's kv head, and the NW partial (max, sum, O) states merge through LDS at the end.
+// Workgroup = 8 waves = U query blocks (32 queries of one q head each) of one kv head x 8 / U key groups. The
+// blocks of a kv head are numbered query block major, so with 2 q heads per kv head a U = 2 workgroup holds both
+// heads' queries of one block. Key group g takes key tiles g, g + 8 / U, ... (32 keys each), staged in LDS once for
+// its U waves; the groups' partial (max, sum, O) states merge through LDS at the end.
 // S^T = K Q^T on f16 MFMA 32x32x16 (products of f16 values are exact in f32, sums in f32): lane (lr, lh) feeds
 // K[key lr][dims 16 s + 8 lh ..] and Q[query lr][same dims], so its accumulator column is query lr with 16 of the
 // tile's keys (8 (r / 4) + 4 lh + r % 4), the other 16 in lane ^ 32; the online softmax runs in f32 on those.
 // O^T = V^T P^T: the B operand of step st is lane's own P values r = 8 st + e, i.e. keys
 // 16 st + 8 (e / 4) + 4 lh + e % 4, fed as two f16 parts (hi = f16(p), lo = f16(p - hi)) so P keeps ~22 bits; the
-// A operand (V^T at those keys) is read from the wave's V tile, transposed into LDS as [dim][key].
+// A operand (V^T at those keys) is read from the row-major V tile by the transposing LDS read.
+// Bound: 2 waves per SIMD (the accumulators and Q fragments take ~200 registers) step through load, MFMA and softmax
+// nearly in phase; T = 2048 on 16 / 8 heads takes 51 us (122 us with V transposed by 2-byte LDS stores and K and V
+// read by every wave for itself), of which the MFMAs alone would be 13. Tried: the next tile's scores under this
+// one's softmax (55), K fragments straight from memory with U = 1 (74 against 66 us).
+typedef h16 half4 __attribute__((ext_vector_type(4)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 constexpr int QHD = 128;
-constexpr int VT_LD = 40;  // keys per V^T row in LDS (32 + 8 pad)
+constexpr int FK_LD = QHD + 8;   // halves per K row in LDS: 16 rows' 16-byte reads fall on all 64 banks
+constexpr int FV_LD = QHD + 32;  // halves per V row: 4 rows' 64-byte pieces (a half wave's read) fall on all 64 banks
+constexpr int FO_LD = QHD + 4;   // floats per query of the merge
 
 struct GqaParams {
   const h16* q;
@@ -691,82 +701,119 @@ struct GqaParams {
   unsigned long long* err;  // the GPU's error record: positions outside the cache
 };
 
-template <int NW>
-__global__ __launch_bounds__(64 * NW) void gqaFlashKernel(GqaParams p) {
-  __shared__ __attribute__((aligned(16))) h16 Vt[NW][QHD * VT_LD];
-  __shared__ float mS[NW][32], lS[NW][32];
-  __shared__ float oS[NW][32][33];
-  const int h = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+// 4 consecutive rows x 16 consecutive halves per 16 lanes, transposed: lane i passes the address of row i / 4,
+// halves 4 (i % 4) .. and gets the 4 rows' values of half i
+__device__ __forceinline__ half4 ldsTranspose4(const h16* a) {
+  typedef short short4v __attribute__((ext_vector_type(4)));
+  typedef __attribute__((address_space(3))) short4v* Lds;
+  return __builtin_bit_cast(half4, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                                       (Lds)(reinterpret_cast<short4v*>(const_cast<h16*>(a)))));
+}
+
+template <int U>
+__global__ __launch_bounds__(512) void gqaFlashKernel(GqaParams p) {
+  constexpr int NS = 8 / U;         // key groups
+  constexpr int BUF = U == 1 ? 1 : 2;  // tiles in LDS per group: a wave alone orders its own stores and reads
+  constexpr int PC = 8 / U;         // 16-byte pieces of a K or V tile per thread of the group
+  constexpr int TILE = 32 * (FK_LD + FV_LD);
+  constexpr int SMEM_T = NS * BUF * TILE * 2, SMEM_O = 8 * 32 * FO_LD * 4;
+  __shared__ __attribute__((aligned(16))) char smem[SMEM_T > SMEM_O ? SMEM_T : SMEM_O];
+  __shared__ float mS[8][32], lS[8][32];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lr = lane & 31, lh = lane >> 5;
+  const int kg = wave / U, ui = wave % U;
+  const int group = static_cast<int>(static_cast<unsigned>(p.qh) / static_cast<unsigned>(p.kvh));
   const int64_t dq = static_cast<int64_t>(p.qh) * QHD, dk = static_cast<int64_t>(p.kvh) * QHD;
-  const int64_t kvOff = static_cast<int64_t>(h / (p.qh / p.kvh)) * QHD;
-  const int64_t q0 = static_cast<int64_t>(blockIdx.x) * 32;
-  const int64_t p0 = *p.pos;
-  const int64_t nk = p0 < 0 ? 0 : min<int64_t>(p0 + p.t, p.cap);  // keys that exist
-  const int64_t qpos = p0 + q0 + lr;                                  // this lane's query position
+  const int kv = static_cast<int>(blockIdx.x % static_cast<unsigned>(p.kvh));  // with 8 kv heads: one XCD's L2 each
+  const int64_t kvOff = static_cast<int64_t>(kv) * QHD;
+  // rows, tiles and blocks in 32 bits: 2^31 rows of a head's 256 bytes are more than the memory
+  const int t = static_cast<int>(p.t), cap = static_cast<int>(p.cap);
+  const int blocks = (t + 31) / 32 * group;  // query blocks of the kv head
+  const auto queryOf = [&](int ub) { return static_cast<int>(static_cast<unsigned>(ub) / static_cast<unsigned>(group)) * 32; };
+  // the longest first: a causal block's work grows with its position
+  const int u0 = static_cast<int>((gridDim.x - 1 - blockIdx.x) / static_cast<unsigned>(p.kvh)) * U, u = u0 + ui;
+  const int64_t pos = *p.pos;
+  const int p0 = pos < 0 ? 0 : pos > cap ? cap : static_cast<int>(pos);  // outside: no query has a row, all NaN below
+  const int nk = pos < 0 ? 0 : (p0 + t < cap ? p0 + t : cap);  // keys that exist
+  const auto tilesOf = [&](int q0) {
+    const int kEnd = p0 + q0 + 32 < nk ? p0 + q0 + 32 : nk;
+    return pos < 0 ? 0 : (kEnd + 31) / 32;
+  };
+  const int q0 = queryOf(u), h = kv * group + u - q0 / 32 * group;
+  const int tiles = u < blocks ? tilesOf(q0) : 0;                             // this wave's
+  const int tilesWg = tilesOf(queryOf((u0 + U < blocks ? u0 + U : blocks) - 1));  // the workgroup's longest: the last's
+  const int qpos = p0 + q0 + lr;  // this lane's query position
   const float sc = p.scale * kLog2e;
   half8 qf[8];
   {
-    const h16* qr = p.q + min<int64_t>(q0 + lr, p.t - 1) * dq + h * QHD + 8 * lh;
+    const h16* qr = p.q + (q0 + lr < t ? q0 + lr : t - 1) * dq + h * QHD + 8 * lh;
 #pragma unroll
     for (int s = 0; s < 8; ++s) qf[s] = ld8(qr + 16 * s);
   }
-  const int64_t kEnd = min<int64_t>(nk, p0 + q0 + 32);
-  const int tiles = kEnd > 0 ? static_cast<int>((kEnd + 31) / 32) : 0;
-  h16* vt = Vt[wave];
+  h16* sm = reinterpret_cast<h16*>(smem) + kg * BUF * TILE;
+  const int gt = tid & (64 * U - 1), gr = gt >> 4, go = gt & 15;  // staging: piece i is row gr + 4 U i, octet go
+  half8 kn[PC], vn[PC];
+  const auto load = [&](int tile) {
+#pragma unroll
+    for (int i = 0; i < PC; ++i) {
+      const int row = tile * 32 + gr + 4 * U * i;
+      const int64_t off = (row < nk ? row : nk - 1) * dk + kvOff + 8 * go;
+      kn[i] = ld8(p.kc + off);
+      vn[i] = ld8(p.vc + off);
+    }
+  };
+  const auto store = [&](int b) {
+    h16* kt = sm + b * TILE;
+    h16* vt = kt + 32 * FK_LD;
+#pragma unroll
+    for (int i = 0; i < PC; ++i) {
+      *reinterpret_cast<half8*>(kt + (gr + 4 * U * i) * FK_LD + 8 * go) = kn[i];
+      *reinterpret_cast<half8*>(vt + (gr + 4 * U * i) * FV_LD + 8 * go) = vn[i];
+    }
+  };
   f32x16 o[4];
 #pragma unroll
   for (int b = 0; b < 4; ++b)
 #pragma unroll
     for (int r = 0; r < 16; ++r) o[b][r] = 0.0f;
-  float m = -INFINITY, l = 0.0f;
-  for (int tile = wave; tile < tiles; tile += NW) {
-    const int64_t k0 = static_cast<int64_t>(tile) * 32;
-    half8 kf[8];
-    const h16* kr = p.kc + min<int64_t>(k0 + lr, nk - 1) * dk + kvOff + 8 * lh;
-#pragma unroll
-    for (int s = 0; s < 8; ++s) kf[s] = ld8(kr + 16 * s);
-    // V tile -> LDS as V^T [dim][key]: lane (key lr, dim octets lh + 2 i)
-    half8 vv[8];
-    const h16* vr = p.vc + min<int64_t>(k0 + lr, nk - 1) * dk + kvOff;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) vv[i] = ld8(vr + 8 * (lh + 2 * i));
+  float m = -INFINITY, l = 0.0f;  // m in units of the raw score
+  const auto compute = [&](int tile, int b) {
+    const h16* kt = sm + b * TILE + lr * FK_LD + 8 * lh;
+    const h16* vt = sm + b * TILE + 32 * FK_LD + (4 * lh + ((lane >> 2) & 3)) * FV_LD + (lane & 16) + 4 * (lane & 3);
     f32x16 s;
 #pragma unroll
     for (int r = 0; r < 16; ++r) s[r] = 0.0f;
 #pragma unroll
-    for (int st = 0; st < 8; ++st) s = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[st], qf[st], s, 0, 0, 0);
+    for (int st = 0; st < 8; ++st) s = __builtin_amdgcn_mfma_f32_32x32x16_f16(ld8(kt + 16 * st), qf[st], s, 0, 0, 0);
+    const int k0 = tile * 32 + 4 * lh;
+    if (tile * 32 + 31 > (nk - 1 < p0 + q0 ? nk - 1 : p0 + q0)) {  // keys past the cache or past some query
+      const int last = (nk - 1 < qpos ? nk - 1 : qpos) - k0;
 #pragma unroll
-    for (int i = 0; i < 8; ++i)
-#pragma unroll
-      for (int e = 0; e < 8; ++e) vt[(8 * (lh + 2 * i) + e) * VT_LD + lr] = vv[i][e];
-    float mt = -INFINITY;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int64_t key = k0 + 8 * (r >> 2) + 4 * lh + (r & 3);
-      s[r] = (key >= nk || key > qpos) ? -INFINITY : s[r] * sc;
-      mt = fmaxf(mt, s[r]);
+      for (int r = 0; r < 16; ++r)
+        if (8 * (r >> 2) + (r & 3) > last) s[r] = -INFINITY;
     }
+    float mt = s[0];
+#pragma unroll
+    for (int r = 1; r < 16; ++r) mt = fmaxf(mt, s[r]);
     mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
-    const float mx = fmaxf(m, mt);
-    const float mn = mx == -INFINITY ? 0.0f : mx;  // a tile wholly past this query: nothing to add
-    const float corr = __builtin_amdgcn_exp2f(m - mn);
+    if (__any(mt > m)) {  // some query's max grew
+      const float mx = fmaxf(m, mt);
+      const float corr = mx == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f((m - mx) * sc);
+      l *= corr;
+      m = mx;
+#pragma unroll
+      for (int bb = 0; bb < 4; ++bb)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[bb][r] *= corr;
+    }
+    const float mn = m == -INFINITY ? 0.0f : m * sc;  // no key up to here: nothing to add
     float ls = 0.0f;
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-      s[r] = __builtin_amdgcn_exp2f(s[r] - mn);
+      s[r] = __builtin_amdgcn_exp2f(fmaf(s[r], sc, -mn));
       ls += s[r];
     }
-    ls += __shfl_xor(ls, 32, 64);
-    l = l * corr + ls;
-    m = mx;
-#pragma unroll
-    for (int b = 0; b < 4; ++b)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) o[b][r] *= corr;
-    // the wave's V^T stores before its reads: LDS serves one wave's operations in order; the fence keeps the
-    // compiler from moving the reads (other lanes' data) above the stores
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    l += ls + __shfl_xor(ls, 32, 64);
 #pragma unroll
     for (int st = 0; st < 2; ++st) {
       half8 ph, pl;
@@ -777,59 +824,106 @@ __global__ __launch_bounds__(64 * NW) void gqaFlashKernel(GqaParams p) {
         pl[e] = static_cast<h16>(v - static_cast<float>(ph[e]));
       }
 #pragma unroll
-      for (int b = 0; b < 4; ++b) {
-        const h16* row = vt + (32 * b + lr) * VT_LD + 16 * st + 4 * lh;
-        half8 va;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          va[e] = row[e];
-          va[4 + e] = row[8 + e];
-        }
-        o[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va, ph, o[b], 0, 0, 0);
-        o[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va, pl, o[b], 0, 0, 0);
+      for (int bb = 0; bb < 4; ++bb) {
+        const half4 v0 = ldsTranspose4(vt + 16 * st * FV_LD + 32 * bb);
+        const half4 v1 = ldsTranspose4(vt + (16 * st + 8) * FV_LD + 32 * bb);
+        const half8 va = __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7);
+        o[bb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va, ph, o[bb], 0, 0, 0);
+        o[bb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va, pl, o[bb], 0, 0, 0);
       }
     }
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");  // this tile's V^T reads before the next tile's stores
-  }
-  // merge the waves, one 32-dim block at a time
-  if (lh == 0) {
-    mS[wave][lr] = m;
-    lS[wave][lr] = l;
+  };
+  if constexpr (U == 1) {
+    if (kg < tiles) load(kg);
+    for (int tile = kg; tile < tiles; tile += NS) {
+      // LDS serves one wave's operations in order; the fences keep the compiler from moving other lanes' data
+      // across its stores
+      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+      store(0);
+      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+      load(tile + NS);  // rows past the end are clamped
+      compute(tile, 0);
+    }
+  } else if (tilesWg > 0) {
+    const int steps = (tilesWg + NS - 1) / NS;
+    load(kg);
+    store(0);
+    load(kg + NS);
+    __syncthreads();
+    for (int j = 0; j < steps; ++j) {
+      store((j + 1) & 1);  // the tile that the last step read; every wave is past it
+      load(kg + (j + 2) * NS);
+      if (kg + j * NS < tiles) compute(kg + j * NS, j & 1);
+      __syncthreads();
+    }
   }
   __syncthreads();
-  constexpr int TPQ = 2 * NW, DPT = 32 / TPQ;  // threads per query, dims per thread and 32-dim block
-  const int q = tid / TPQ, d0 = (tid % TPQ) * DPT;
+  // merge the key groups
+  float* oS = reinterpret_cast<float*>(smem);
+  if (kg < tiles) {
+    if (lh == 0) {
+      mS[wave][lr] = m;
+      lS[wave][lr] = l;
+    }
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+#pragma unroll
+      for (int r = 0; r < 16; r += 4)
+        *reinterpret_cast<f32x4*>(oS + (wave * 32 + lr) * FO_LD + 32 * b + 2 * r + 4 * lh) =
+            f32x4{o[b][r], o[b][r + 1], o[b][r + 2], o[b][r + 3]};
+  }
+  __syncthreads();
+  constexpr int TPQ = 16 / U;  // threads per query
+  const int mu = tid / (512 / U), q = tid % (512 / U) / TPQ, d0 = tid % TPQ * 4;
+  const int mb = u0 + mu;  // the block that this thread merges
+  if (mb >= blocks) return;
+  const int qb = queryOf(mb), qrow = qb + q, hm = kv * group + mb - qb / 32 * group;
+  if (qrow >= t) return;
+  const int used = tilesOf(qb);  // key groups beyond it had no tile
   float mxw = -INFINITY;
 #pragma unroll
-  for (int w = 0; w < NW; ++w) mxw = fmaxf(mxw, mS[w][q]);
-  float scw[NW], wsum = 0.0f;
+  for (int w = 0; w < NS; ++w)
+    if (w < used) mxw = fmaxf(mxw, mS[w * U + mu][q]);
+  float scw[NS], wsum = 0.0f;
 #pragma unroll
-  for (int w = 0; w < NW; ++w) {
-    scw[w] = lS[w][q] > 0.0f ? __builtin_amdgcn_exp2f(mS[w][q] - mxw) : 0.0f;
-    wsum += scw[w] * lS[w][q];
+  for (int w = 0; w < NS; ++w) {
+    const float lw = w < used ? lS[w * U + mu][q] : 0.0f;
+    scw[w] = lw == 0.0f ? 0.0f : __builtin_amdgcn_exp2f((mS[w * U + mu][q] - mxw) * sc);
+    wsum += scw[w] * lw;
   }
   const float inv = 1.0f / wsum;
-  const int64_t qrow = q0 + q;
-  const bool noRow = p0 + qrow >= p.cap || p0 < 0;
+  const bool noRow = pos < 0 || p0 + qrow >= cap;
   // recorded once, by the thread of head 0 that owns the first query without a cache row
-  if (noRow && qrow < p.t && d0 == 0 && blockIdx.y == 0 && qrow == (p0 < 0 ? 0 : p.cap - p0))
-    raiseDeviceError(p.err, LK_DEVERR_POSITION, p0 + qrow);
+  if (noRow && d0 == 0 && hm == 0 && pos <= cap && qrow == (pos < 0 ? 0 : cap - p0))
+    raiseDeviceError(p.err, LK_DEVERR_POSITION, pos + qrow);
+  h16* orow = p.out + qrow * dq + hm * QHD;
+  const bool outVec = (reinterpret_cast<uintptr_t>(p.out) & 7) == 0;
 #pragma unroll
-  for (int b = 0; b < 4; ++b) {
+  for (int i = 0; i < QHD / (4 * TPQ); ++i) {
+    const int d = d0 + 4 * TPQ * i;
+    f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+    half4 y;
+    const auto add = [&](int w) {
+      const f32x4 v = *reinterpret_cast<const f32x4*>(oS + ((w * U + mu) * 32 + q) * FO_LD + d);
 #pragma unroll
-    for (int r = 0; r < 16; ++r) oS[wave][lr][8 * (r >> 2) + 4 * lh + (r & 3)] = o[b][r];
-    __syncthreads();
-    if (qrow < p.t) {
-      h16* orow = p.out + qrow * dq + h * QHD + 32 * b + d0;
+      for (int e = 0; e < 4; ++e) acc[e] = fmaf(scw[w], v[e], acc[e]);
+    };
+    if (used >= NS) {  // apart, so that its reads are issued together
 #pragma unroll
-      for (int d = 0; d < DPT; ++d) {
-        float acc = 0.0f;
+      for (int w = 0; w < NS; ++w) add(w);
+    } else {
 #pragma unroll
-        for (int w = 0; w < NW; ++w) acc += scw[w] * oS[w][q][d0 + d];
-        orow[d] = noRow ? static_cast<h16>(__builtin_nanf("")) : toH16(acc * inv);
-      }
+      for (int w = 0; w < NS; ++w)
+        if (w < used) add(w);
     }
-    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < 4; ++e) y[e] = noRow ? static_cast<h16>(__builtin_nanf("")) : toH16(acc[e] * inv);
+    if (outVec) {
+      *reinterpret_cast<half4*>(orow + d) = y;
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) orow[d + e] = y[e];
+    }
   }
 }
 
@@ -1530,10 +1624,16 @@ int lk_hip_f16_attention_gqa(const void* q, const void* kc, const void* vc, cons
     hipLaunchKernelGGL(gqaDecodeMergeKernel, dim3(static_cast<unsigned>(qh)), dim3(128), 0, s, p);
     return launched();
   }
-  // 8 waves per 32-query block: a causal block holds few key tiles, so more waves in flight per block
-  // (Qwen3 416-id prefill 3.94 -> 3.89 ms against 4)
-  hipLaunchKernelGGL(gqaFlashKernel<8>, dim3(static_cast<unsigned>((t + 31) / 32), static_cast<unsigned>(qh)),
-                     dim3(512), 0, s, p);
+  // Two query blocks per workgroup halve the K / V reads and staging per block, and the workgroups; they pay once
+  // the halved grid still holds one workgroup per CU (LDS admits one). us by (T, q heads / kv heads), one block
+  // against two: (416, 16/8) 11.3 / 13.7; (800, 16/8) 19.8 / 20.0; (1024, 16/8) 24.1 / 22.7; (500, 32/8) 17.2 / 14.8;
+  // (2048, 16/8) 65.8 / 50.8; (4000, 16/8) 193 / 156. (Both heads' V transposed by 2-byte LDS stores, each wave its
+  // own tiles: 13.8, 30.3, 42.1, 25.9, 122, 320.)
+  const int64_t blocks = (t + 31) / 32 * (qh / kvh);
+  if (blocks * kvh >= 512)
+    hipLaunchKernelGGL(gqaFlashKernel<2>, dim3(static_cast<unsigned>((blocks + 1) / 2 * kvh)), dim3(512), 0, s, p);
+  else
+    hipLaunchKernelGGL(gqaFlashKernel<1>, dim3(static_cast<unsigned>(blocks * kvh)), dim3(512), 0, s, p);
   return launched();
 }
 

@@ -195,6 +195,37 @@ def test_attention_gqa_small_group_counts(gpu):
             check(got, X.attention_gqa(q, kc, vc, pos, qh, kvh), extra, f"gqa {qh}/{kvh} t={t}")
 
 
+# one query block per workgroup below 512 blocks over all kv heads, two from there on: block counts that are odd, head
+# groups of 1, 2, 3 and 4, tiles cut by the end of the prompt, fewer and more tiles than key groups. The cache rows
+# past the prompt hold NaN: none of them may enter a result.
+@pytest.mark.parametrize("t,pos,qh,kvh", [(31, 0, 3, 1), (32, 1, 16, 8), (257, 0, 16, 8), (993, 0, 16, 8),
+                                          (992, 0, 16, 8), (333, 31, 48, 16), (257, 300, 64, 64), (300, 1, 64, 16)])
+def test_attention_gqa_blocks(gpu, t, pos, qh, kvh):
+    lk = gpu
+    q, kc, vc = _attn_case(t, pos, qh, kvh, pos + t + 40)
+    kc[pos + t:], vc[pos + t:] = np.nan, np.nan
+    got = lk.ops.f16_gpu.attention_gqa_opt_f16_gpu(G(lk, q), G(lk, kc), G(lk, vc), P(lk, pos), q_heads=qh, kv_heads=kvh)
+    extra = 2.0 ** -22 * (8 + np.sqrt(pos + t)) * np.abs(O.c(vc[:pos + t])).max()
+    check(got, X.attention_gqa(q, kc, vc, pos, qh, kvh), extra, f"gqa {qh}/{kvh} t={t} pos={pos}")
+
+
+# the same rule on both sides for queries without a cache row, at the cache's end and wholly past it
+@pytest.mark.parametrize("t,pos", [(40, 30), (1100, 30), (1100, 64), (1100, 5000)])
+def test_attention_gqa_blocks_past_the_cache(gpu, t, pos):
+    lk = gpu
+    cap = 64
+    q, kc, vc = _attn_case(t, pos, 16, 8, cap)
+    out = lk.ops.f16_gpu.attention_gqa_opt_f16_gpu(G(lk, q), G(lk, kc), G(lk, vc), P(lk, pos))
+    fit = max(cap - pos, 0)
+    if pos <= cap:
+        with pytest.raises(LokinferError, match=f"device error 2.*detail {max(pos, cap)}"):
+            check_device_errors()
+    got = out.numpy().astype(np.float64)
+    if fit:
+        check(got[:fit], X.attention_gqa(q[:fit], kc, vc, pos, 16, 8), 2.0 ** -22 * 16 * np.abs(O.c(vc)).max(), "fit")
+    assert np.isnan(got[fit:]).all()
+
+
 def test_rows_past_the_cache(gpu):
     lk = gpu
     F = lk.ops.f16_gpu
