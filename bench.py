@@ -30,7 +30,7 @@ HBM_PEAK_GBS = 8000.0
 # LayerNorms; the tied LM head (wte); ln_f; the token and position rows; K and V rows 0..512 of 12 layers (f32)
 GPT2_STEP_BYTES = 4 * (12 * (768 * 2304 + 768 * 768 + 2 * 768 * 3072 + 2304 + 768 + 3072 + 768 + 4 * 768)
                        + 50257 * 768 + 2 * 768 + 2 * 768 + 12 * 2 * 513 * 768)
-F32_MFMA_PEAK_TFLOPS = 157.3
+BF16_MFMA_PEAK_TFLOPS = 2500.0
 
 
 def event_times(fn, n: int) -> list[float]:
@@ -282,9 +282,10 @@ def wino_tiles(lo: int, d: int, m: int = 4) -> int:
 
 
 def roofline_wino(launches: int = 20, calibrate: bool = False) -> dict:
-    """The dominant kernel of the Kokoro forward: the Winograd GEMM (winoMmKernel<4,7,3,3>, wino_mm_lc_f32_gpu with
-    U tiled, u_layout 1, as the Kokoro graph runs it) of a generator stage-1 resblock conv (L = 120 F + 1 rows at 487 tokens, 128 -> 128 channels, K = 11 as 3 nested
-    F(4,4) tap groups, d = 5). Its algorithm is A = 7 point GEMMs over (group, channel): 2 A T (N Ci) Co FLOPs
+    """The dominant kernel of the Kokoro forward: the Winograd GEMM (winoMmKernel<4,7,3>, wino_mm_lc_f32_gpu with
+    U in its bf16 parts, u_layout 2, as the Kokoro graph runs it) of a generator stage-1 resblock conv (L = 120 F + 1 rows at 487 tokens, 128 -> 128 channels, K = 11 as 3 nested
+    F(4,4) tap groups, d = 5). Each f32 product is six bf16 MFMA products (the operands in three exact bf16 parts),
+    so the peak is the bf16 one over 6. Its algorithm is A = 7 point GEMMs over (group, channel): 2 A T (N Ci) Co FLOPs
     per launch for T output tiles of 4 rows. The whole conv (input transform + GEMM, snake prologue) is timed
     beside it and reported against the direct conv's 2 L Ci Co K FLOPs. With calibrate, also launches add_f32_gpu
     over 2^26 floats (reads 512 MiB, writes 256 MiB) as the reference kernel for the --pmc byte counters."""
@@ -302,9 +303,10 @@ def roofline_wino(launches: int = 20, calibrate: bool = False) -> dict:
     _, n = W.variant(k)
     attrs = dict(dilation=d, groups=n, kernel=k, padding=pad, tile=4)
     v = lk.ops.wino_tf_lc_f32_gpu(x, tr, affine=af, alpha=alpha, **attrs)
-    mm = lambda: lk.ops.wino_mm_lc_f32_gpu(v, u, b, tr, x, u_layout=1, **attrs)  # noqa: E731
+    u = lk.ops.wino_split_u_f32_gpu(u)
+    mm = lambda: lk.ops.wino_mm_lc_f32_gpu(v, u, b, tr, x, u_layout=2, **attrs)  # noqa: E731
     conv = lambda: lk.ops.conv1d_wino_lc_f32_gpu(x, u, b, tr, k, padding=pad, dilation=d, affine=af,  # noqa: E731
-                                                 alpha=alpha, u_layout=1)
+                                                 alpha=alpha, u_layout=2)
     mm()
     ms = statistics.mean(event_times(mm, launches))
     conv()
@@ -319,10 +321,11 @@ def roofline_wino(launches: int = 20, calibrate: bool = False) -> dict:
     a = W.alpha_of(k)
     flops = 2.0 * a * wino_tiles(l, d) * (n * c) * c
     direct = 2.0 * l * c * c * k
-    return {"kernel": "winoMmKernel<4,7,3,3,1,true> (wino_mm_lc_f32_gpu, tiled U: K = 11 Winograd GEMM, "
-                      "generator stage 1)",
-            "bound": "mfma", "achieved": flops / (ms * 1e-3) / 1e12, "peak": F32_MFMA_PEAK_TFLOPS,
-            "unit": "TFLOP/s", "frac": flops / (ms * 1e-3) / 1e12 / F32_MFMA_PEAK_TFLOPS,
+    peak = BF16_MFMA_PEAK_TFLOPS / 6
+    return {"kernel": "winoMmKernel<4,7,3> (wino_mm_lc_f32_gpu, U in bf16 parts: K = 11 Winograd GEMM, "
+                      "generator stage 1; peak = bf16 MFMA / 6 products)",
+            "bound": "mfma", "achieved": flops / (ms * 1e-3) / 1e12, "peak": peak,
+            "unit": "TFLOP/s", "frac": flops / (ms * 1e-3) / 1e12 / peak,
             "traffic": measured_traffic(), "avg_launch_ms": ms, "flops_per_launch": flops,
             "conv_ms": conv_ms, "conv_direct_equiv_tflops": direct / (conv_ms * 1e-3) / 1e12}
 

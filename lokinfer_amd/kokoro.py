@@ -205,7 +205,8 @@ class KokoroGpu:
         Winograd pair or the tap conv, whichever is faster at this shape. Measured on MI355X over every conv of the
         59- and 487-token forwards: the pair (transform + GEMM) costs at least ~55-60 us, the K = 3 tap conv ~55-60
         us per 1e9 multiply-adds, and K >= 7 favours Winograd once its grid of 64-tile x 64-channel workgroups
-        reaches 64. co_pad > Co: output channels past Co are zero (zero weights and bias). Returns (y, stats,
+        reaches 64 (timed with the pair's GEMM on f32 MFMAs; on bf16 parts it already wins from 0.47e9 at K = 3, but
+        there its error, 1.3e-6 against float64, is above the tap conv's 5e-7). co_pad > Co: output channels past Co are zero (zero weights and bias). Returns (y, stats,
         stats_dilation): Winograd statistics come per residue class of the dilation."""
         co, ci = self.sd[p + ".weight"].shape[:2]
         cop = max(co, co_pad)
