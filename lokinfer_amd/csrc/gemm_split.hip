@@ -188,13 +188,13 @@ __global__ __launch_bounds__(64 * NW * KG) void gemmWsKernel(GemmWsParams p) {
   for (int t = 0; t < D - 1; ++t)
     if (s + t < maxSteps) step(sb + s + t, t & 1 ? st1 : st0, t & 1 ? st0 : st1, ra[(t + 1) % D], rb[t]);
 
-  // a non-finite or overflowing operand leaves NaN: such a wave sums its K range again on f32 MFMAs
-  float nan = 0.0f;
+  // an infinity or NaN may come from the split (split3.h): such a wave sums its K range again on f32 MFMAs
+  float bad = 0.0f;
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) nan += acc[i][r] += low[i][r];
-  if (__any(nan != nan)) {
+    for (int r = 0; r < 16; ++r) bad = fmaf(acc[i][r] += low[i][r], 0.0f, bad);  // NaN after either
+  if (__any(bad != bad)) {
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll

@@ -8,8 +8,9 @@
 // values are off by 1.6e-7 / 4.3e-7 / 9.5e-7 (2-norm) at K = 128 / 768 / 3072, on f32 MFMAs by 2.1e-7 / 4.9e-7 / 1.0e-6.
 //
 // An infinite or NaN element, or one that rounds past the largest bf16, splits into parts of which one is NaN, and so
-// makes every output it enters NaN: kernels test their outputs for NaN and recompute such tiles on f32 MFMAs, which
-// gives the value the f32 sum has. The bf16 MFMAs flush denormal parts: elements below about 2^-110 keep fewer than
+// makes every output it enters NaN; two finite elements whose product f32 still holds may have h h' past it (both round
+// up), which leaves an infinity. Kernels test their sums for either and recompute such tiles on f32 MFMAs, which gives the
+// value the f32 sum has. The bf16 MFMAs flush denormal parts: elements below about 2^-110 keep fewer than
 // 24 bits.
 #pragma once
 

@@ -334,14 +334,14 @@ __global__ __launch_bounds__(256, 3) void winoMmKernel(WinoMmArgs p) {
   }
   if (s < se) step(s, As0, As1, ra1);
 
-  // a non-finite or overflowing operand leaves NaN in every output it enters: such a wave runs its steps again on
-  // f32 MFMAs, operands straight from memory
-  float nan = 0.0f;
+  // an infinity or NaN may come from the split (split3.h): such a wave runs its steps again on f32 MFMAs, operands
+  // straight from memory
+  float bad = 0.0f;
 #pragma unroll
   for (int j = 0; j < M; ++j)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) nan += y[j][r];
-  if (__any(nan != nan)) {
+    for (int r = 0; r < 16; ++r) bad = fmaf(y[j][r], 0.0f, bad);  // NaN after either
+  if (__any(bad != bad)) {
 #pragma unroll
     for (int j = 0; j < M; ++j) clear(y[j]);
 #pragma unroll 1

@@ -91,3 +91,31 @@ def test_gemm_ws_refuses(lk):
     with pytest.raises(ValueError):
         lk.ops.gemm_ws_f32_gpu(G(lk, np.ones((2, 8))), w)
     assert lk.ops.gemm_ws_f32_gpu(G(lk, np.ones((0, 16))), w).shape == (0, 4)
+
+
+# one shape per kernel of the launcher's rule: 32 x 32 with K over eight waves, 32 x 64 over two and four wave groups,
+# 32 x 128 and 64 x 128 tiles
+KERNELS = [(33, 40, 70), (487, 768, 768), (487, 2056, 768), (1024, 48, 2304), (8200, 64, 1056)]
+
+
+def _products(lk, a, w, planes):
+    """a w, by one launch or as the sum of `planes` K ranges (each entry of the tests that use it is one product)."""
+    ws = lk.ops.split_weight(G(lk, w))
+    if planes == 1:
+        return lk.ops.gemm_ws_f32_gpu(G(lk, a), ws).numpy()
+    with np.errstate(all="ignore"):
+        return lk.ops.gemm_ws_splitk_f32_gpu(G(lk, a), ws, planes).numpy().sum(0)
+
+
+@pytest.mark.parametrize("m,k,n,planes", [s + (1,) for s in KERNELS] + [(59, 256, 96, 4)])
+def test_gemm_ws_largest_products(lk, m, k, n, planes):
+    """A product that f32 holds is not lost where the operands' leading parts, both rounded up, multiply past it."""
+    top = np.float32(0.9985 * 2.0 ** 64)
+    a, w = np.zeros((m, k), np.float32), np.zeros((k, n), np.float32)
+    want = np.zeros((m, n), np.float32)
+    for i, (row, col, kk) in enumerate([(0, 0, 0), (m // 2, n // 3, k // 2), (m - 1, n - 1, k - 1)]):
+        a[row, kk] = top * np.float32(2.0 ** (20 * i))
+        w[kk, col] = top * np.float32(-2.0 ** (-20 * i))
+        want[row, col] = a[row, kk] * w[kk, col]
+    assert np.isfinite(want).all() and np.abs(want).max() > 3.39e38
+    assert np.array_equal(_products(lk, a, w, planes), want)

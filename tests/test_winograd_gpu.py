@@ -329,3 +329,57 @@ def test_wino_mm_extreme_operands(gpu, ci, l, k, layout):
         assert np.isfinite(got[ok]).all()
         inf = np.isinf(ref)
         assert np.array_equal(got[inf], ref[inf].astype(np.float32))
+
+
+def _mm_operands(lk, r, ci, l, k, tile, d, layout, u=None):
+    """A wino_mm call over random operands of 64 output channels: (run(v, u), v, u, tr, exact(v, u)); run launches it
+    in the given u_layout, exact is the same in float64."""
+    n, a, m = W.variant(k)[1], W.alpha_of(k, tile), 2 if tile == 2 else 4
+    tr = W.wino_weights(np.zeros((64, 16, k)), tile)[1]
+    rows = W.tiles_rows(l, d, n, tile, k)
+    v = r.standard_normal((rows, ci)).astype(np.float32)
+    u = r.standard_normal((a, n * ci, 64)).astype(np.float32)
+    x, zero = np.zeros((l, ci), np.float32), np.zeros(64, np.float32)
+    at = tr[a * a:].astype(np.float64).reshape(m, a)
+
+    def run(v, u):
+        dev = G(lk, u if layout == 0 else W.tile_u(u, n))
+        dev = lk.ops.wino_split_u_f32_gpu(dev) if layout == 2 else dev
+        return lk.ops.wino_mm_lc_f32_gpu(G(lk, v), dev, G(lk, zero), G(lk, tr), G(lk, x), dilation=d, groups=n, kernel=k,
+                                         padding=_pad(k, d), tile=tile, u_layout=layout).numpy()
+
+    def exact(v, u, at=at):
+        v, u = v.astype(np.float64).reshape(d, a, -1, ci), u.astype(np.float64)
+        y = np.zeros((l, 64))
+        for rho in range(min(d, l)):
+            t = -(-len(range(rho, l, d)) // m)
+            p = [sum(v[rho, i, g:g + t] @ u[i, g * ci:(g + 1) * ci] for g in range(n)) for i in range(a)]
+            full = np.stack([sum(at[j, i] * p[i] for i in range(a)) for j in range(m)], 1).reshape(m * t, 64)
+            y[rho::d] = full[:len(range(rho, l, d))]
+        return y
+
+    def bound(v, u):  # of the f32 sum: n ci products per point, A points, random signs
+        return 2.0 ** -24 * (6 + 2 * np.sqrt(n * ci * a)) * exact(np.abs(v), np.abs(u), np.abs(at))
+
+    return run, v, u, exact, bound
+
+
+# every kernel of the launcher: tile 2, one to three chunks of 16 channels per step, two and three tap groups; split-K
+# (one residue of a few tiles), dilation
+MM_KERNELS = [(32, 200, 3, 2, 1), (16, 90, 3, 4, 2), (32, 300, 3, 4, 1), (48, 300, 3, 4, 3), (32, 200, 7, 4, 3),
+              (48, 150, 11, 4, 1), (768, 70, 3, 4, 1)]
+
+
+@pytest.mark.parametrize("layout", [0, 1, 2])
+@pytest.mark.parametrize("ci,l,k,tile,d", MM_KERNELS)
+def test_wino_mm_largest_products(gpu, ci, l, k, tile, d, layout):
+    """A product that f32 holds is not lost where the operands' leading parts, both rounded up, multiply past it."""
+    run, v, u, exact, _ = _mm_operands(gpu, np.random.default_rng(1), ci, l, k, tile, d, layout)
+    v, u = np.zeros_like(v), np.zeros_like(u)
+    top = np.float32(0.9985 * 2.0 ** 64)
+    r1 = len(v) // (d * len(u))  # the rows of point 1 (residue 0), whose coefficients AT[:, 1] are all 1
+    v[r1 + 3, 5], v[r1 + 10, ci - 1] = top, -top
+    u[1, 5, 7], u[1, ci - 1, 40] = top, top
+    want = exact(v, u).astype(np.float32)
+    assert np.isfinite(want).all() and np.abs(want).max() > 3.39e38
+    assert np.array_equal(run(v, u), want)
