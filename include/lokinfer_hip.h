@@ -250,8 +250,9 @@ int lk_hip_wino_mm_ut_lc_f32(const float* v, const float* ut, const float* bias,
                              int dilation, int groups, int kernel, int tile, float scale, void* workspace,
                              int64_t workspace_bytes, void* stream);
 /* The same with U given split (MI355X backend; the wino_mm ops' u_layout = 2): us bf16 [A, Co / 64, 2, Ci / 16, N, 3,
- * 64, 8], the three bf16 parts whose sum is U in the order of the kernel's matrix fragments (lk_hip_wino_split_u_f32);
- * the same bits again. */
+ * 64, 8], the three bf16 parts whose sum is U in the order of the kernel's matrix fragments (lk_hip_wino_split_u_f32; an
+ * element under 2^-110 that they cannot hold is a NaN part and its own bits); the same bits again, except where a tile is
+ * recomputed in f32: sums past 2^82 (u, ut) or 2^105 (us), and the columns of such elements. */
 int lk_hip_wino_mm_us_lc_f32(const float* v, const void* us, const float* bias, const float* res, float* out,
                              const float* tr, float* stats, int64_t v_rows, int64_t ci, int64_t co, int64_t lo,
                              int dilation, int groups, int kernel, int tile, float scale, void* workspace,
@@ -266,7 +267,7 @@ int lk_hip_wino_adain_affine_lc_f32(const float* stats, const float* gb, float* 
 
 /* ---- f32 GEMM over split weights (MI355X backend): the weight in three exact bf16 parts, laid out once in
  *      matrix-fragment order, the products on the bf16 matrix cores at f32 precision ---- */
-/* w f32[K, N] (nt = 0) or f32[N, K] (nt = 1) -> ws, ceil(N / 32) ceil(K / 16) 3072 bytes */
+/* w f32[K, N] (nt = 0) or f32[N, K] (nt = 1) -> ws, ceil(N / 32) ceil(K / 16) 3072 bytes (parts of every float, as us) */
 int lk_hip_split_weight_f32(const float* w, void* ws, int64_t n, int64_t k, int nt, void* stream);
 /* out[M, N] = (act(a[M, K] W + bias) + res) * scale (act 0 none, 1 ReLU, 2 gelu_tanh; bias, res optional); K % 8 == 0,
  * a and ws 16-byte aligned */

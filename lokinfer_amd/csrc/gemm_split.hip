@@ -193,7 +193,10 @@ __global__ __launch_bounds__(64 * NW * KG) void gemmWsKernel(GemmWsParams p) {
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) bad = fmaf(acc[i][r] += low[i][r], 0.0f, bad);  // NaN after either
+    for (int r = 0; r < 16; ++r) {
+      acc[i][r] = (acc[i][r] + low[i][r]) * kSplitUnscale;
+      bad = fmaf(acc[i][r], 0.0f, bad);  // NaN after either
+    }
   if (__any(bad != bad)) {
 #pragma unroll
     for (int i = 0; i < TM; ++i)

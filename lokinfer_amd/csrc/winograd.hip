@@ -263,11 +263,11 @@ __global__ __launch_bounds__(256, 3) void winoMmKernel(WinoMmArgs p) {
 #pragma unroll
     for (int r = 0; r < 16; ++r) x[r] = 0.0f;
   };
-  // a finished point (or this split's part of it) folds into the output rows
-  auto fold = [&](int xi) {
+  // a finished point (or this split's part of it), its sums in units of 1 / unit, folds into the output rows
+  auto fold = [&](int xi, float unit) {
 #pragma unroll
     for (int j = 0; j < M; ++j) {
-      const float at = p.tr[A * A + j * A + xi];
+      const float at = p.tr[A * A + j * A + xi] * unit;
 #pragma unroll
       for (int r = 0; r < 16; ++r) y[j][r] += at * acc[r];
     }
@@ -322,7 +322,7 @@ __global__ __launch_bounds__(256, 3) void winoMmKernel(WinoMmArgs p) {
       loadB(up, e, rb[e]);  // the next step's
     }
     const bool wrap = cs + 1 == chunks;
-    if (wrap || s == se - 1) fold(xs);
+    if (wrap || s == se - 1) fold(xs, UL == 2 ? kSplitUnscale : kSplitUnscale * kSplitUnscale);
     cs = wrap ? 0 : cs + 1;
     xs += wrap;
     __syncthreads();
@@ -361,7 +361,7 @@ __global__ __launch_bounds__(256, 3) void winoMmKernel(WinoMmArgs p) {
           for (int q = 0; q < 4; ++q) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(aq[q], bq[h][q], acc, 0, 0, 0);
         }
       }
-      if (cf == chunks - 1 || f == se - 1) fold(xf);
+      if (cf == chunks - 1 || f == se - 1) fold(xf, 1.0f);
     }
   }
 

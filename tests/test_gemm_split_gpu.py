@@ -119,3 +119,32 @@ def test_gemm_ws_largest_products(lk, m, k, n, planes):
         want[row, col] = a[row, kk] * w[kk, col]
     assert np.isfinite(want).all() and np.abs(want).max() > 3.39e38
     assert np.array_equal(_products(lk, a, w, planes), want)
+
+
+@pytest.mark.parametrize("m,k,n,planes", [s + (1,) for s in KERNELS] + [(59, 256, 96, 4)])
+@pytest.mark.parametrize("small", ["a", "w"])
+def test_gemm_ws_small_operands(lk, m, k, n, planes, small):
+    """Operands down to the smallest denormals, in rows of A or columns of W, enter with all their bits."""
+    r = np.random.default_rng(m + k + n)
+    a, w = r.standard_normal((m, k)) * 2.0 ** 60, r.standard_normal((k, n)) * 2.0 ** 60
+    down = 2.0 ** -r.integers(160, 208, m if small == "a" else n)  # 2^-100 .. 2^-147
+    a, w = (a * down[:, None], w) if small == "a" else (a, w * down)
+    a, w = a.astype(np.float32), w.astype(np.float32)
+    ref = a.astype(np.float64) @ w
+    bound = 2.0 ** -24 * (4 + np.sqrt(k)) * (np.abs(a).astype(np.float64) @ np.abs(w))  # f32 sums of k products
+    assert (np.abs(_products(lk, a, w, planes) - ref) <= bound).all()
+
+
+def test_split_weight_parts(lk):
+    """Every element is the sum of its parts, or, where three bf16 parts cannot hold it, stored whole behind a NaN."""
+    r = np.random.default_rng(9)
+    w = (r.standard_normal((64, 96)) * 2.0 ** r.integers(-149, 100, (64, 96))).astype(np.float32)
+    w[0, :4] = [0.0, -0.0, 2.0 ** -149, -(2.0 ** -110 - 2.0 ** -134)]
+    p = lk.ops.split_weight(G(lk, w)).ws.numpy().view(np.uint16).reshape(3, 4, 3, 2, 32, 8).astype(np.uint32)
+    p = p.transpose(2, 1, 3, 5, 0, 4).reshape(3, 64, 96)  # part, (chunk, half, k), (block, column)
+    f = (p << 16).view(np.float32)
+    whole = np.isnan(f[0])
+    assert whole.any() and (np.abs(w[whole]) < 2.0 ** -110).all()
+    with np.errstate(invalid="ignore"):
+        back = np.where(whole, (p[1] << 16 | p[2]).view(np.float32), (f[0] + f[1]) + f[2])
+    assert np.array_equal(back, w)

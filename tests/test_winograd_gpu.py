@@ -383,3 +383,17 @@ def test_wino_mm_largest_products(gpu, ci, l, k, tile, d, layout):
     want = exact(v, u).astype(np.float32)
     assert np.isfinite(want).all() and np.abs(want).max() > 3.39e38
     assert np.array_equal(run(v, u), want)
+
+
+@pytest.mark.parametrize("layout", [0, 1, 2])
+@pytest.mark.parametrize("ci,l,k,tile,d", MM_KERNELS)
+def test_wino_mm_small_operands(gpu, ci, l, k, tile, d, layout):
+    """Operands down to the smallest denormals, all of V or columns of U, enter with all their bits."""
+    r = np.random.default_rng(ci + l + k)
+    run, v, u, exact, bound = _mm_operands(gpu, r, ci, l, k, tile, d, layout)
+    big = np.float32(2.0 ** 60)
+    for e in (-112, -127, -145):
+        tiny = (v * 2.0 ** e).astype(np.float32)
+        assert (np.abs(run(tiny, u * big) - exact(tiny, u * big)) <= bound(tiny, u * big)).all()
+    tiny = (u * 2.0 ** -r.integers(100, 148, 64)).astype(np.float32)
+    assert (np.abs(run(v * big, tiny) - exact(v * big, tiny)) <= bound(v * big, tiny)).all()
