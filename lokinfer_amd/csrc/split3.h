@@ -119,6 +119,7 @@ __device__ __forceinline__ void splitExact(const float (&v)[8], u32x4 (&parts)[3
       part[q] = (cut || !finite ? b : b + 0x7fff + ((b >> 16) & 1)) >> 16;
       rest = finite ? rest - __uint_as_float(part[q] << 16) : 0.0f;
     }
+    if (v[k] != v[k]) part[0] |= 0x40;  // a NaN whose bits are all in the low half
     if (rest != 0.0f) {
       const unsigned b = __float_as_uint(v[k]);
       part[0] = 0x7fc0;

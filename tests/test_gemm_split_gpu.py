@@ -148,3 +148,13 @@ def test_split_weight_parts(lk):
     with np.errstate(invalid="ignore"):
         back = np.where(whole, (p[1] << 16 | p[2]).view(np.float32), (f[0] + f[1]) + f[2])
     assert np.array_equal(back, w)
+
+
+@pytest.mark.parametrize("m,k,n", KERNELS)
+def test_gemm_ws_nan_weights(lk, m, k, n):
+    """Every NaN stays one when a weight is laid out, also with all its significand bits in the low half."""
+    r = np.random.default_rng(3)
+    a, w = r.standard_normal((m, k)).astype(np.float32), r.standard_normal((k, n)).astype(np.float32)
+    w.view(np.uint32)[1, 2], w.view(np.uint32)[k - 1, n - 1] = 0x7f800001, 0xff800001
+    y = lk.ops.gemm_ws_f32_gpu(G(lk, a), lk.ops.split_weight(G(lk, w))).numpy()
+    assert np.isnan(y[:, [2, n - 1]]).all() and np.isfinite(np.delete(y, [2, n - 1], 1)).all()

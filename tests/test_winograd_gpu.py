@@ -397,3 +397,12 @@ def test_wino_mm_small_operands(gpu, ci, l, k, tile, d, layout):
         assert (np.abs(run(tiny, u * big) - exact(tiny, u * big)) <= bound(tiny, u * big)).all()
     tiny = (u * 2.0 ** -r.integers(100, 148, 64)).astype(np.float32)
     assert (np.abs(run(v * big, tiny) - exact(v * big, tiny)) <= bound(v * big, tiny)).all()
+
+
+@pytest.mark.parametrize("layout", [0, 1, 2])
+def test_wino_mm_nan_weights(gpu, layout):
+    """Every NaN of U stays one, also with all its significand bits in the low half (the split layout)."""
+    run, v, u, _, _ = _mm_operands(gpu, np.random.default_rng(2), 32, 200, 3, 4, 1, layout)
+    u.view(np.uint32)[1, 7, 5], u.view(np.uint32)[2, 31, 60] = 0x7f800001, 0xff800001
+    y = run(v, u)
+    assert np.isnan(y[:, [5, 60]]).all() and np.isfinite(np.delete(y, [5, 60], 1)).all()
