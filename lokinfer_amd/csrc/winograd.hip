@@ -242,7 +242,7 @@ __global__ __launch_bounds__(256, 3) void winoMmKernel(WinoMmArgs p) {
 #pragma unroll
       for (int h = 0; h < 2; ++h)
 #pragma unroll
-        for (int q = 0; q < 4; ++q) r[h][q] = ue[(4 * h + q) * co + boff];
+        for (int q = 0; q < 4; ++q) r[h][q] = ue[static_cast<int64_t>(4 * h + q) * co + boff];
     } else {
 #pragma unroll
       for (int h = 0; h < (UL == 1 ? 2 : 3); ++h)
@@ -367,18 +367,30 @@ __global__ __launch_bounds__(256, 3) void winoMmKernel(WinoMmArgs p) {
 
   // Register r = tile tb0 + 8 (r / 4) + 4 lk + r % 4, channel c0 + bcol. Output rows go through buffer resources that
   // end with the tensor (a row past the residue class is past the tensor): loads there give 0 and stores are dropped,
-  // with no branch per element. One resource per 8-tile row group keeps the lane offsets in 32 bits.
+  // with no branch per element. One resource per 8-tile row group keeps the lane offsets in 32 bits; rows too long for
+  // that (32 of them past 4 GB) are addressed one by one.
   const int64_t tb0 = t0 + 32 * __builtin_amdgcn_readfirstlane(wm);
   const int left = static_cast<int>(min<int64_t>(lor - tb0 * M, 32 * M)) - 4 * lk * M;  // output rows from this lane's
   auto orow = [&](int j, int r) { return (8 * (r >> 2) + (r & 3)) * M + j; };
-  const unsigned rowBytes = static_cast<unsigned>(d * co) * 4;
+  const int64_t stride = static_cast<int64_t>(d) * co;
+  const bool wide = stride >= int64_t{1} << 25;
+  const unsigned rowBytes = static_cast<unsigned>(stride) * 4;
   const unsigned ooff = 4 * lk * M * rowBytes + static_cast<unsigned>(c0 + bcol) * 4;
   auto rows = [&](const float* base, int rg) {  // the 8-tile group rg
     const int64_t first = rho + (tb0 + 8 * rg) * M * d;
     const int64_t bytes = base ? min<int64_t>(max<int64_t>(p.lo - first, 0) * co * 4, 0xfffffff0) : 0;
     return uniformRsrc(base + (bytes ? first * co : 0), static_cast<unsigned>(bytes));
   };
+  const int64_t wideOff = rho * static_cast<int64_t>(co) + (tb0 + 4 * lk) * M * stride + c0 + bcol;
   auto store = [&](float* base) {
+    if (wide) {
+#pragma unroll
+      for (int j = 0; j < M; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          if (orow(j, r) < left) base[wideOff + orow(j, r) * stride] = y[j][r];
+      return;
+    }
 #pragma unroll
     for (int rg = 0; rg < 4; ++rg) {
       const auto rs = rows(base, rg);
@@ -402,10 +414,15 @@ __global__ __launch_bounds__(256, 3) void winoMmKernel(WinoMmArgs p) {
 #pragma unroll
   for (int j = 0; j < M; ++j) {
     float rv[16];
+    if (wide) {
 #pragma unroll
-    for (int r = 0; r < 16; ++r)
-      rv[r] = __uint_as_float(
-          __builtin_amdgcn_raw_buffer_load_b32(rs[r >> 2], ooff + ((r & 3) * M + j) * rowBytes, 0, 0));
+      for (int r = 0; r < 16; ++r) rv[r] = p.res && orow(j, r) < left ? p.res[wideOff + orow(j, r) * stride] : 0.0f;
+    } else {
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        rv[r] = __uint_as_float(
+            __builtin_amdgcn_raw_buffer_load_b32(rs[r >> 2], ooff + ((r & 3) * M + j) * rowBytes, 0, 0));
+    }
 #pragma unroll
     for (int r = 0; r < 16; ++r) y[j][r] = ((y[j][r] + bias) + rv[r]) * p.scale;
     __builtin_amdgcn_sched_barrier(0);
@@ -551,7 +568,8 @@ int winoMm(const float* v, const float* u, const float* bias, const float* res, 
   // measured slower than no split on MI355X: the partial rows' round trip and the second launch outweigh the extra
   // workgroups; so did splits up to three workgroups per CU at 16 steps), partials in the workspace past its 64 KiB
   // counter area
-  if (static_cast<int64_t>(dilation) * co >= int64_t{1} << 25) return 1;  // 32 output rows within 32-bit offsets
+  // lane offsets of 32 bits: 66 rows of V, 8 rows of U (operands of more than 150 GB)
+  if ((63 + groups) * ci >= int64_t{1} << 32 || 8 * co >= int64_t{1} << 32) return 1;
   const int64_t base = (co / 64) * ((tiles + 63) / 64) * dilation;
   const int steps = a * static_cast<int>(ci / 16);  // in 16-channel units
   // one tap group: 48 or 32 channels per pipeline step where they divide Ci (with more groups the second chunk's

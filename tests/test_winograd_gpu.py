@@ -406,3 +406,33 @@ def test_wino_mm_nan_weights(gpu, layout):
     u.view(np.uint32)[1, 7, 5], u.view(np.uint32)[2, 31, 60] = 0x7f800001, 0xff800001
     y = run(v, u)
     assert np.isnan(y[:, [5, 60]]).all() and np.isfinite(np.delete(y, [5, 60], 1)).all()
+
+
+@pytest.mark.parametrize("layout", [0, 1, 2])
+def test_wino_mm_wide_rows(gpu, layout):
+    """Output rows of which 32 take 4 GB (dilation x Co = 2^25): a column block gives the same bits as by itself."""
+    import torch
+
+    lk, ci, co, d, l = gpu, 16, 1 << 19, 64, 270  # 4 or 5 rows per residue class
+    g = torch.Generator(device="cuda").manual_seed(7)
+    rnd = lambda *s: torch.randn(*s, device="cuda", generator=g)  # noqa: E731
+    tr = lk.Tensor(torch.from_numpy(W.wino_weights(np.zeros((64, 16, 3)))[1]).cuda())
+    v, u, b, res = rnd(W.tiles_rows(l, d, 1, 4, 3), ci), rnd(6, ci, co), rnd(co), rnd(l, co)
+    x = lk.Tensor(torch.zeros(l, ci, device="cuda"))
+
+    def run(cols):
+        n = cols.stop - cols.start
+        w = u[:, :, cols]
+        if layout:  # winograd.tile_u
+            w = w.reshape(6, ci // 16, 4, 4, n // 64, 64).permute(0, 4, 1, 2, 5, 3).reshape(6, n // 64, ci * 64)
+        w = lk.Tensor(w.contiguous())
+        w = lk.ops.wino_split_u_f32_gpu(w) if layout == 2 else w
+        y, st = lk.ops.wino_mm_lc_f32_gpu(lk.Tensor(v), w, lk.Tensor(b[cols]), tr, x, dilation=d, groups=1, kernel=3,
+                                          padding=d, tile=4, residual=lk.Tensor(res[:, cols]), out_scale=0.5, stats=True,
+                                          u_layout=layout)
+        return y.t, st.t
+
+    y, st = run(slice(0, co))
+    for c in (0, co // 2, co - 128):
+        yc, sc = run(slice(c, c + 128))
+        assert torch.equal(y[:, c:c + 128], yc) and torch.equal(st[:, c:c + 128], sc)
