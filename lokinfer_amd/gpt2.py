@@ -141,7 +141,13 @@ class Gpt2Generator(Gpt2Decoder):
     """Chunked prefill + decode sharing the caches (reference build_generate, models/gpt2.py:250-333). sk: split-K
     factors of the two N = 768 projections for T > 1 ((0, 0) = one sum + add_bias_layernorm2). chunk_graph:
     capture each chunk length's forward as a HIP graph (pays off when one length recurs; a one-off prompt runs
-    eagerly)."""
+    eagerly).
+
+    The chunk forward's projections run over split weights, a second copy of 6 bytes per element (0.51 GB beside the
+    0.50 GB of f32 weights, which the decode step streams; a program that only ever steps single tokens can use
+    Gpt2Decoder). The copy follows `w`: a chunk lays out again, in place, every weight that torch counts a write to (or
+    that was replaced) since. Writes that torch does not count (through `.data`, or by another library's pointer) need
+    a `split_weights()` call of their own."""
 
     def __init__(self, sd: dict[str, np.ndarray], graph: bool = True, fused: bool = True, sk=(2, 4),
                  chunk_graph: bool = False):
@@ -149,10 +155,24 @@ class Gpt2Generator(Gpt2Decoder):
         self.sk = tuple(sk)
         dev = self.w["transformer.wte.weight"].t.device
         self.positions = torch.arange(N_POS, dtype=torch.int64, device=dev)  # device pos views, no host copies
-        # the chunk forward's projections run over split weights (the decode step streams the plain ones)
-        self.ws = {k: ops.split_weight(v) for k, v in self.w.items()
-                   if k.endswith(("attn.c_attn.weight", "attn.c_proj.weight", "mlp.c_fc.weight", "mlp.c_proj.weight"))}
+        self.ws: dict[str, ops.SplitWeight] = {}
+        self._laid: dict[str, tuple] = {}  # the torch tensor behind each split weight and its version when laid out
+        self.split_weights()
         self.chunk_model = lk_capture(self._chunk, graph=chunk_graph)
+
+    def split_weights(self, written_only: bool = False) -> None:
+        """Lays the chunk forward's split weights out from `w`: all of them, or those written since the last time."""
+        capturing = torch.cuda.is_current_stream_capturing()
+        for k, v in self.w.items():
+            if not k.endswith(("attn.c_attn.weight", "attn.c_proj.weight", "mlp.c_fc.weight", "mlp.c_proj.weight")):
+                continue
+            version = None if v.t.is_inference() else v.t._version  # an inference tensor has no count: laid out anew
+            laid = self._laid.get(k)
+            if written_only and laid is not None and laid[0] is v.t and version is not None and laid[1] == version:
+                continue
+            self.ws[k] = ops.split_weight(v, out=self.ws.get(k))
+            # while a graph is captured the copy is only recorded: the next eager call still has to make it
+            self._laid[k] = (v.t, None if capturing else version)
 
     def _chunk(self, ids: Tensor, pos: Tensor):
         w = self.w
@@ -196,6 +216,7 @@ class Gpt2Generator(Gpt2Decoder):
         p = Tensor(self.positions[pos:pos + 1])
         if T == 1:
             return self.step(ids, p)
+        self.split_weights(written_only=True)
         return self.chunk_model.run_inplace(ids, p)
 
     def __call__(self, ids, pos: int):

@@ -249,11 +249,15 @@ class SplitWeight:
         self.ws, self.shape = ws, tuple(shape)
 
 
-def split_weight(w, nt: bool = False) -> SplitWeight:
-    """(MI355X backend) w f32[K, N] (nt: f32[N, K]) -> SplitWeight, laid out once for the gemm_ws ops."""
+def split_weight(w, nt: bool = False, out: SplitWeight | None = None) -> SplitWeight:
+    """(MI355X backend) w f32[K, N] (nt: f32[N, K]) -> SplitWeight, laid out once for the gemm_ws ops; `out`: into
+    that one's memory (a weight of the same shape, after it was written)."""
     _f32(w, rank=2)
     k, n = (w.shape[1], w.shape[0]) if nt else w.shape
-    return SplitWeight(_launch("split_weight_f32_gpu", [w], [(-(-n // 32), -(-k // 16) * 768)], dict(nt=int(nt))), (k, n))
+    check(out is None or out.shape == (k, n), "out must be a SplitWeight of the same (K, N)")
+    ws = _launch("split_weight_f32_gpu", [w], [(-(-n // 32), -(-k // 16) * 768)], dict(nt=int(nt)),
+                 outs=None if out is None else [out.ws])
+    return SplitWeight(ws, (k, n))
 
 
 def gemm_ws_f32_gpu(a, w: SplitWeight, bias=None, act="none", residual=None):

@@ -116,3 +116,31 @@ def test_capture_with_collectable_models(setup):
     b = G.Gpt2Generator(sd, graph=False)
     b([5, 6, 7], 0)
     assert np.array_equal(la, b([8], 3))
+
+
+@pytest.mark.parametrize("chunk_graph", [False, True])
+def test_chunks_follow_written_weights(setup, chunk_graph):
+    """The prompt chunk runs on the weights as they are, like the decode step: after an in-place write its logits are a
+    fresh model's, and after a second one, and when a weight's tensor was replaced."""
+    import torch
+
+    G, O, sd, m = setup
+    ids = np.random.default_rng(6).integers(0, G.VOCAB, 90).astype(np.int64)
+    model = G.Gpt2Generator(sd, chunk_graph=chunk_graph)
+    first = model(ids, 0)
+    new, fc, proj = dict(sd), "transformer.h.3.mlp.c_fc.weight", "transformer.h.0.attn.c_attn.weight"
+    for step in range(3):
+        for k, f in ((fc, 1.5), (proj, -0.5)):
+            new[k] = new[k] * np.float32(f)
+            if step == 0:
+                model.w[k].t.mul_(f)
+            elif step == 1:
+                with torch.inference_mode():
+                    model.w[k].t.copy_(torch.from_numpy(new[k]))
+            elif not chunk_graph:
+                model.w[k] = type(model.w[k])(torch.from_numpy(new[k]).to(model.w[k].t.device))
+            else:
+                model.w[k].t.data.copy_(torch.from_numpy(new[k]))
+                model.split_weights()
+        got = model(ids, 0)
+        assert np.array_equal(got, G.Gpt2Generator(new)(ids, 0)) and not np.array_equal(got, first)
