@@ -163,6 +163,7 @@ class Gpt2Generator(Gpt2Decoder):
     def split_weights(self, written_only: bool = False) -> None:
         """Lays the chunk forward's split weights out from `w`: all of them, or those written since the last time."""
         capturing = torch.cuda.is_current_stream_capturing()
+        laid_out = False
         for k, v in self.w.items():
             if not k.endswith(("attn.c_attn.weight", "attn.c_proj.weight", "mlp.c_fc.weight", "mlp.c_proj.weight")):
                 continue
@@ -173,6 +174,9 @@ class Gpt2Generator(Gpt2Decoder):
             self.ws[k] = ops.split_weight(v, out=self.ws.get(k))
             # while a graph is captured the copy is only recorded: the next eager call still has to make it
             self._laid[k] = (v.t, None if capturing else version)
+            laid_out = True
+        if laid_out and not capturing:  # like an uploaded weight: ready for every stream that may run first
+            torch.cuda.current_stream().synchronize()
 
     def _chunk(self, ids: Tensor, pos: Tensor):
         w = self.w

@@ -117,9 +117,16 @@ class KokoroGpu:
         k = key + "#split"
         if k not in self._g:
             with untraced():
-                self._g[k] = ops.split_weight(from_numpy(np.ascontiguousarray(make(), np.float32), device="gpu", copy=True),
-                                              nt=True)
+                ws = ops.split_weight(from_numpy(np.ascontiguousarray(make(), np.float32), device="gpu", copy=True), nt=True)
+            self._laid_out()
+            self._g[k] = ws
         return self._g[k]
+
+    @staticmethod
+    def _laid_out() -> None:
+        """Waits for a weight laid out on the current stream before it is shared: like an uploaded one, it may be used
+        next on another stream or thread."""
+        torch.cuda.current_stream().synchronize()
 
     def _bank(self, root: str):
         """All `<root>.*.fc` style projections as one [128, total] weight (one GEMV per style vector), with each
@@ -196,6 +203,7 @@ class KokoroGpu:
             u, tr = winograd.wino_weights_t(wp)
             with untraced():
                 us = ops.wino_split_u_f32_gpu(from_numpy(u, device="gpu", copy=True))
+            self._laid_out()
             self._g[k] = (us, from_numpy(tr, device="gpu", copy=True))
         return self._g[k]
 

@@ -144,3 +144,23 @@ def test_chunks_follow_written_weights(setup, chunk_graph):
                 model.split_weights()
         got = model(ids, 0)
         assert np.array_equal(got, G.Gpt2Generator(new)(ids, 0)) and not np.array_equal(got, first)
+
+
+def test_split_weights_ready_on_any_stream(setup, monkeypatch):
+    """A model built on one stream, where laying a weight out takes long, runs at once on another."""
+    import torch
+
+    G, O, sd, m = setup
+    ids = np.random.default_rng(8).integers(0, G.VOCAB, 40).astype(np.int64)
+    want = G.Gpt2Generator(sd)(ids, 0)
+    lay = G.ops.split_weight
+
+    def late(*a, **kw):
+        torch.cuda._sleep(20_000_000)  # some 10 ms on the device
+        return lay(*a, **kw)
+
+    monkeypatch.setattr(G.ops, "split_weight", late)
+    with torch.cuda.stream(torch.cuda.Stream()):
+        model = G.Gpt2Generator(sd)
+    with torch.cuda.stream(torch.cuda.Stream()):
+        assert np.array_equal(model(ids, 0), want)

@@ -164,3 +164,33 @@ def test_conv1d_1ch(gpu):
     ref = F.conv1d(torch.from_numpy(x).double()[None, None], torch.from_numpy(w).double()[None, None],
                    torch.from_numpy(b).double(), stride=2, padding=1)[0, 0].numpy()
     close(lk.ops.conv1d_1ch_f32_gpu(G(lk, x), G(lk, w), G(lk, b), stride=2, padding=1), ref, 1e-6)
+
+
+def test_laid_out_weights_ready_on_any_stream(gpu, monkeypatch):
+    """A weight first laid out on one stream, where that takes long, is used at once on another."""
+    from lokinfer_amd import kokoro as M
+
+    lk = gpu
+    w, c = rng.standard_normal((96, 64)).astype(np.float32), rng.standard_normal((64, 32, 3)).astype(np.float32)
+    m = M.KokoroGpu.__new__(M.KokoroGpu)  # the weight cache alone
+    m._g, m.sd = {}, {"c.weight": c}
+    a = G(lk, rng.standard_normal((40, 64)))
+    want_w = lk.ops.gemm_ws_f32_gpu(a, lk.ops.split_weight(G(lk, w), nt=True)).numpy()
+    want_u = m.wino("c.weight", 32, 64)[0].numpy()
+    m._g.clear()
+
+    def late(f):
+        def call(*args, **kw):
+            torch.cuda._sleep(100_000_000)  # some 50 ms on the device
+            return f(*args, **kw)
+        return call
+
+    monkeypatch.setattr(M.ops, "split_weight", late(M.ops.split_weight))
+    monkeypatch.setattr(M.ops, "wino_split_u_f32_gpu", late(M.ops.wino_split_u_f32_gpu))
+    with torch.cuda.stream(torch.cuda.Stream()):
+        ws, us = m.split_w("w", lambda: w), m.wino("c.weight", 32, 64)[0]
+    with torch.cuda.stream(torch.cuda.Stream()):
+        got_w, got_u = lk.ops.gemm_ws_f32_gpu(a, ws), us.t.clone()
+        torch.cuda.current_stream().synchronize()
+        assert np.array_equal(got_w.numpy(), want_w)
+        assert np.array_equal(got_u.cpu().numpy().view(np.uint32), want_u.view(np.uint32))
