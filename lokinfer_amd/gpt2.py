@@ -187,6 +187,8 @@ class Gpt2Generator(Gpt2Decoder):
         ln = ops.layernorm_f32_gpu(h, w[P + "h.0.ln_1.weight"], w[P + "h.0.ln_1.bias"], eps=LN_EPS)
 
         def proj_ln(x, wk, res, ln_key, splits):  # (res + x @ W + b, LN of it)
+            if splits:
+                ops.check_splits(x.shape[1], splits)
             if splits and ops.splitk_planes(T, D, splits) > 1:
                 parts = ops.gemm_ws_splitk_f32_gpu(x, self.ws[wk + "weight"], splits)
                 return ops.add_bias_layernorm2_sk_f32_gpu(parts, w[wk + "bias"], res, w[ln_key + "weight"],

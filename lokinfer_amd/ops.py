@@ -714,10 +714,14 @@ def attention_gen2_f32_gpu(qkv, kcache, vcache, pos, bias, heads):
     return _cache_attn("attention_gen2_f32_gpu", qkv, kcache, vcache, pos, bias, heads, dict(heads=int(heads)))
 
 
+def check_splits(k: int, splits) -> None:
+    check(int(splits) >= 1 and k % (16 * int(splits)) == 0, "K must be divisible by 16*splits")
+
+
 def _splitk_check(a, b, splits, tile):
     _f32(a, b, rank=2)
     check(a.shape[1] == b.shape[0], "inner dimensions differ")
-    check(int(splits) >= 1 and a.shape[1] % (16 * int(splits)) == 0, "K must be divisible by 16*splits")
+    check_splits(a.shape[1], splits)
     check(int(tile) in (32, 64), "tile must be 32 or 64")
     check(b.shape[1] % 4 == 0, "N must be a multiple of 4")
     return (int(splits), a.shape[0], b.shape[1])

@@ -164,3 +164,13 @@ def test_split_weights_ready_on_any_stream(setup, monkeypatch):
         model = G.Gpt2Generator(sd)
     with torch.cuda.stream(torch.cuda.Stream()):
         assert np.array_equal(model(ids, 0), want)
+
+
+@pytest.mark.parametrize("sk", [(5, 4), (2, 7), (-1, 4), (2, -4)])
+def test_refuses_split_factors(setup, sk):
+    """Split-K factors that do not divide K into multiples of 16 are refused at every chunk length."""
+    G, O, sd, m = setup
+    model = G.Gpt2Generator(sd, sk=sk)
+    for t in (2, 40, 700):
+        with pytest.raises(G.ops.OpError):
+            model(np.zeros(t, np.int64), 0)
