@@ -295,35 +295,46 @@ int gemmWs(const float* a, const void* ws, const float* bias, const float* res, 
   if (m == 0 || n == 0) return 0;
   const lkd::GemmWsParams p{a, static_cast<const lkd::u32x4*>(ws), bias, res, out, m, n, k, act, scale, planes};
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const int64_t rows = lkh::ceilDiv(m, 32);
-  const int64_t g2 = rows * lkh::ceilDiv(n, 64);
   const auto go = [&](auto kernel, int tm, int nw, int kg) {
     hipLaunchKernelGGL(kernel, dim3(lkh::ceilDiv(n, 32 * nw), lkh::ceilDiv(m, 32 * tm), static_cast<unsigned>(planes)),
                        dim3(64 * nw * kg), 0, s, p);
   };
-  // The largest tile whose grid still fills the 256 CUs, K over more waves where none does. Times in us (graph replay)
-  // at (M, K, N): gemm.hip's f32 MFMA kernels (with their split-K reduction), this rule's choice, others
-  //   64 x 128 tiles, from 1024 of them: (48880, 256, 1536) 384, 258. (4888, 512, 5120) 278, 160
-  //   32 x 128, from 512: (1024, 768, 2304) 63, 33; 64 x 128 37
-  //   32 x 64 with K over two wave groups, from 160: (487, 768, 2304) 31.3, 20.8; one group 22.3, 32 x 128 23.1.
-  //     (512, 768, 3072) 31.0, 22.6; 22.5 at 32 x 128. (487, 768, 768) 14.0, 11.4
-  //   32 x 64 over four groups for long K on such a grid: (487, 2048, 768) 28.8, 20.9; two groups 22.8. (512, 3072, 768)
-  //     35.2, 28.4; 31.7
-  //   32 x 32 with K over eight waves: (59, 768, 2304) 10.8, 9.0; 32 x 64 over two 11.2. (59, 768, 768) 9.9, 8.8.
-  //     (200, 2048, 768) 19.1, 14.0; 22.3. (59, 2048, 768) 11.7, 13.7: the one shape where the f32 kernels, eight
-  //     workgroups along K, are ahead (before the partial planes they leave to the LayerNorm)
-  if (planes > 1)
-    go(lkd::gemmWsKernel<1, 1, 8, 16, 4>, 1, 1, 8);
-  else if (static_cast<int64_t>(lkh::ceilDiv(m, 64)) * lkh::ceilDiv(n, 128) >= 1024)
-    go(lkd::gemmWsKernel<2, 4, 1, 32, 2>, 2, 4, 1);
-  else if (rows * lkh::ceilDiv(n, 128) >= 512)
-    go(lkd::gemmWsKernel<1, 4, 1, 32, 4>, 1, 4, 1);
-  else if (g2 >= 160 && g2 < 256 && k >= 2048)
-    go(lkd::gemmWsKernel<1, 2, 4, 32, 2>, 1, 2, 4);
-  else if (g2 >= 160)
+  // Workgroups with tiles of 32 x 32, 32 x 64, 32 x 128 and 64 x 128. Smaller tiles read A and B more often, larger ones
+  // leave CUs idle, so the rule is the smallest tile that fits the chip in one round of workgroups: one to each of the 256
+  // CUs where K is spread over the waves (eight waves), then as many as the registers admit, three or two of four waves;
+  // beyond that the largest tile. In us (graph replay) at (M, K, N), gemm.hip's f32 MFMA kernels (with their split-K
+  // reduction), then the forms around the line:
+  //   32 x 32 | 32 x 64, K over eight / four waves: (96, 768, 2304) 13.4, 8.3 | 9.8; (128, 768, 2304) 13.5, 17.0 | 10.0;
+  //     (320, 768, 768) 18.0, 14.0 | 15.0; (360, 768, 768) 18.5, 19.9 | 15.2
+  //   32 x 64 | 32 x 128 over two: (200, 768, 2304) 13.7, 10.2 | 12.5; (256, 768, 2304) 20.5, 14.4 | 13.6; (600, 2048, 768)
+  //     39.8, 26.0 | 34.4; (700, 2048, 768) 49.7, 35.3 | 34.8
+  //   32 x 128 over two | 32 x 64 over two with four waves: (430, 768, 2304) 23.0, 14.5 | 16.5; (460, 768, 2304) 28.4, 21.8
+  //     | 20.5; (600, 768, 2048) 31.3, 23.6 | 22.6
+  //   32 x 64 over two | 32 x 128: (512, 768, 3072) 32.1, 26.1 | 27.7; (600, 768, 3072) 40.9, 32.0 | 27.9; (900, 768, 2048)
+  //     40.5, 31.2 | 26.0
+  //   32 x 128 | 64 x 128: (1200, 256, 1536) 19.7, 11.9 | 12.4; (2400, 256, 1536) 41.2, 22.0 | 18.7; (800, 512, 5120) 64.1,
+  //     33.7 | 40.7 (520 of the larger tiles: a second round for 8 of them); (1200, 512, 5120) 86.8, 51.1 | 44.3; (48880, 256,
+  //     1536) 328, - | 268
+  // One block of rows leaves most CUs without a workgroup and waits for W: four waves that load four steps ahead instead of
+  // eight that load two, W from memory: (32, 768, 2304) 11.4 against 12.0, f32 10.9; (32, 3072, 768) in four ranges 18.1
+  // against 18.8, f32 19.6; W in the caches 8.5 against 7.7, f32 10.1. Narrow W keeps the eight: (32, 768, 768) 11.9, 12.7.
+  const int64_t rows = static_cast<int64_t>(lkh::ceilDiv(m, 32)) * planes;
+  const int64_t g1 = rows * lkh::ceilDiv(n, 32), g2 = rows * lkh::ceilDiv(n, 64), g4 = rows * lkh::ceilDiv(n, 128);
+  const int64_t g8 = static_cast<int64_t>(lkh::ceilDiv(m, 64)) * lkh::ceilDiv(n, 128) * planes;
+  if (m <= 32 && g1 > 64 && g1 <= 256)
+    go(lkd::gemmWsKernel<1, 1, 4, 16, 4>, 1, 1, 4);
+  else if (g1 <= 256)
+    go(lkd::gemmWsKernel<1, 1, 8, 16, 2>, 1, 1, 8);
+  else if (g2 <= 256)
+    go(lkd::gemmWsKernel<1, 2, 4, 16, 2>, 1, 2, 4);
+  else if (g4 <= 256)
+    go(lkd::gemmWsKernel<1, 4, 2, 32, 2>, 1, 4, 2);
+  else if (g2 <= 768)
     go(lkd::gemmWsKernel<1, 2, 2, 32, 2>, 1, 2, 2);
+  else if (g4 <= 512 || (g4 <= 1024 && g8 > 512))
+    go(lkd::gemmWsKernel<1, 4, 1, 32, 4>, 1, 4, 1);
   else
-    go(lkd::gemmWsKernel<1, 1, 8, 16, 4>, 1, 1, 8);
+    go(lkd::gemmWsKernel<2, 4, 1, 32, 2>, 2, 4, 1);
   return hipGetLastError() == hipSuccess ? 0 : 2;
 }
 

@@ -16,13 +16,16 @@ def G(lk, a):
     return lk.from_numpy(np.ascontiguousarray(a, np.float32), device="gpu", copy=True)
 
 
-# (M, K, N): one kernel of the launcher's rule each (64 x 128 tiles, 32 x 128, 32 x 64 with K over two / four wave groups,
-# 32 x 32 over eight), with ragged rows, columns and K tails, K shorter than the wave groups, single rows and columns
+# (M, K, N): ragged rows, columns and K tails, K shorter than the wave groups, single rows and columns
 SHAPES = [(1, 8, 1), (1, 16, 33), (31, 24, 32), (33, 40, 31), (59, 768, 2304), (200, 2048, 96), (487, 768, 768),
           (500, 72, 700), (487, 2056, 770), (1030, 136, 2100), (4100, 40, 2090), (8200, 256, 1056)]
+# one per kernel of the launcher's rule: 32 x 32 with K over eight and four waves, 32 x 64 over four and two wave
+# groups, 32 x 128 over two and one, 64 x 128; the second half with one step or none for some of the groups
+KERNELS = [(33, 776, 70), (31, 264, 2100), (487, 776, 768), (500, 136, 2304), (430, 264, 2300), (640, 48, 2990),
+           (1500, 72, 2304), (32, 16, 2080), (600, 8, 768), (1000, 24, 700), (700, 40, 1300)]
 
 
-@pytest.mark.parametrize("m,k,n", SHAPES)
+@pytest.mark.parametrize("m,k,n", SHAPES + KERNELS)
 def test_gemm_ws(lk, m, k, n):
     r = np.random.default_rng(m + 3 * k + 7 * n)
     a, w = r.standard_normal((m, k)).astype(np.float32), r.standard_normal((k, n)).astype(np.float32)
@@ -72,7 +75,8 @@ def test_gemm_ws_extreme_operands(lk, m, k, n):
                 assert (np.abs(got[fits] - ref[fits]) <= bound[fits]).all()
 
 
-@pytest.mark.parametrize("m,k,n,s", [(1, 64, 40, 3), (2, 16, 31, 5), (59, 2048, 768, 4), (320, 136, 700, 7), (400, 256, 768, 4)])
+@pytest.mark.parametrize("m,k,n,s", [(1, 64, 40, 3), (2, 16, 31, 5), (59, 2048, 768, 4), (320, 136, 700, 7), (400, 256, 768, 4),
+                                     (32, 264, 700, 4), (100, 264, 768, 4), (256, 136, 768, 4), (300, 72, 760, 6)])
 def test_gemm_ws_splitk(lk, m, k, n, s):
     r = np.random.default_rng(m + k)
     a, w = r.standard_normal((m, k)).astype(np.float32), r.standard_normal((k, n)).astype(np.float32)
@@ -93,11 +97,6 @@ def test_gemm_ws_refuses(lk):
     assert lk.ops.gemm_ws_f32_gpu(G(lk, np.ones((0, 16))), w).shape == (0, 4)
 
 
-# one shape per kernel of the launcher's rule: 32 x 32 with K over eight waves, 32 x 64 over two and four wave groups,
-# 32 x 128 and 64 x 128 tiles
-KERNELS = [(33, 40, 70), (487, 768, 768), (487, 2056, 768), (1024, 48, 2304), (8200, 64, 1056)]
-
-
 def _products(lk, a, w, planes):
     """a w, by one launch or as the sum of `planes` K ranges (each entry of the tests that use it is one product)."""
     ws = lk.ops.split_weight(G(lk, w))
@@ -107,7 +106,7 @@ def _products(lk, a, w, planes):
         return lk.ops.gemm_ws_splitk_f32_gpu(G(lk, a), ws, planes).numpy().sum(0)
 
 
-@pytest.mark.parametrize("m,k,n,planes", [s + (1,) for s in KERNELS] + [(59, 256, 96, 4)])
+@pytest.mark.parametrize("m,k,n,planes", [s + (1,) for s in KERNELS] + [(59, 256, 96, 4), (256, 136, 768, 4)])
 def test_gemm_ws_largest_products(lk, m, k, n, planes):
     """A product that f32 holds is not lost where the operands' leading parts, both rounded up, multiply past it."""
     top = np.float32(0.9985 * 2.0 ** 64)
@@ -121,7 +120,7 @@ def test_gemm_ws_largest_products(lk, m, k, n, planes):
     assert np.array_equal(_products(lk, a, w, planes), want)
 
 
-@pytest.mark.parametrize("m,k,n,planes", [s + (1,) for s in KERNELS] + [(59, 256, 96, 4)])
+@pytest.mark.parametrize("m,k,n,planes", [s + (1,) for s in KERNELS] + [(59, 256, 96, 4), (256, 136, 768, 4)])
 @pytest.mark.parametrize("small", ["a", "w"])
 def test_gemm_ws_small_operands(lk, m, k, n, planes, small):
     """Operands down to the smallest denormals, in rows of A or columns of W, enter with all their bits."""
