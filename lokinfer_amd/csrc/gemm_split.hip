@@ -93,7 +93,7 @@ __global__ __launch_bounds__(64 * NW * KG) void gemmWsKernel(GemmWsParams p) {
   const int ik = static_cast<int>(p.k);
   const int64_t lastRow = p.m - 1;
 
-  // A units of this thread: 8 consecutive k of one row; k past K loads the row's start and is zeroed when split
+  // A units of this thread: 4 UF consecutive k of one row; k past K loads the row's start and is zeroed when split
   const float* arow[UA];
   int aslot[UA], ak[UA];
 #pragma unroll
@@ -119,21 +119,21 @@ __global__ __launch_bounds__(64 * NW * KG) void gemmWsKernel(GemmWsParams p) {
   };
   auto storeA = [&](Stage* st, int s, const f32x4(&r)[UA][UF]) {
     // zero past K, and past the range of a group with fewer steps than the others: its products add nothing, and no
-    // load or MFMA sits behind a branch (which would make the compiler wait for the loads just issued)
+    // load or MFMA sits behind a branch (which would make the compiler wait for the loads just issued). The zero is the
+    // split's scale, so it takes no instruction of its own (an infinity there becomes NaN, but its row holds one as well).
     const int k0 = s < se ? s * KS : ik;
 #pragma unroll
     for (int u = 0; u < UA; ++u) {
-      const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-      const int kk = k0 + ak[u];
+      const float scale = k0 + ak[u] < ik ? kSplitScale : 0.0f;  // K % 8 == 0: a unit ends within K or starts past it
       if constexpr (UF == 2) {
-        const Frag3 f = split3(kk < ik ? r[u][0] : zero, kk + 4 < ik ? r[u][1] : zero);
+        const Frag3 f = split3(r[u][0], r[u][1], scale);
         u32x4* dst = &st[kg][0][0][0] + aslot[u];
         dst[0] = __builtin_bit_cast(u32x4, f.h);
         dst[BM * 2] = __builtin_bit_cast(u32x4, f.m);
         dst[2 * BM * 2] = __builtin_bit_cast(u32x4, f.l);
       } else {
         u32x2* dst = reinterpret_cast<u32x2*>(&st[kg][0][0][0]) + aslot[u];
-        split3(kk < ik ? r[u][0] : zero, dst[0], dst[BM * 4], dst[2 * BM * 4]);
+        split3(r[u][0], scale, dst[0], dst[BM * 4], dst[2 * BM * 4]);
       }
     }
   };

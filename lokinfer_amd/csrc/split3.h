@@ -30,13 +30,14 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 
-constexpr float kSplitScale = 0x1p23f;    // of the parts that split3 makes
+constexpr float kSplitScale = 0x1p23f;     // of the parts that split3 makes
 constexpr float kSplitUnscale = 0x1p-23f;  // of a sum with one such operand; squared with two
 
-// the parts of kSplitScale a and kSplitScale b as bf16 pairs (a in the low half)
-__device__ __forceinline__ void split3(float a, float b, unsigned& h, unsigned& m, unsigned& l) {
-  a *= kSplitScale;
-  b *= kSplitScale;
+// the parts of scale a and scale b (scale kSplitScale, or 0 for elements past the operand's end) as bf16 pairs (a in the
+// low half)
+__device__ __forceinline__ void split3(float a, float b, float scale, unsigned& h, unsigned& m, unsigned& l) {
+  a *= scale;
+  b *= scale;
   h = __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2{a, b}), bf16x2));
   const float ra = a - __uint_as_float(h << 16), rb = b - __uint_as_float(h & 0xffff0000u);
   m = __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2{ra, rb}), bf16x2));
@@ -45,10 +46,10 @@ __device__ __forceinline__ void split3(float a, float b, unsigned& h, unsigned& 
                                        bf16x2));
 }
 
-__device__ __forceinline__ void split3(f32x4 x, u32x2& h, u32x2& m, u32x2& l) {
+__device__ __forceinline__ void split3(f32x4 x, float scale, u32x2& h, u32x2& m, u32x2& l) {
   unsigned a[3], b[3];
-  split3(x[0], x[1], a[0], a[1], a[2]);
-  split3(x[2], x[3], b[0], b[1], b[2]);
+  split3(x[0], x[1], scale, a[0], a[1], a[2]);
+  split3(x[2], x[3], scale, b[0], b[1], b[2]);
   h = u32x2{a[0], b[0]};
   m = u32x2{a[1], b[1]};
   l = u32x2{a[2], b[2]};
@@ -59,10 +60,10 @@ struct Frag3 {
   bf16x8 h, m, l;
 };
 
-__device__ __forceinline__ Frag3 split3(f32x4 x0, f32x4 x1) {
+__device__ __forceinline__ Frag3 split3(f32x4 x0, f32x4 x1, float scale) {
   u32x2 h0, m0, l0, h1, m1, l1;
-  split3(x0, h0, m0, l0);
-  split3(x1, h1, m1, l1);
+  split3(x0, scale, h0, m0, l0);
+  split3(x1, scale, h1, m1, l1);
   return Frag3{__builtin_bit_cast(bf16x8, (u32x4{h0[0], h0[1], h1[0], h1[1]})),
                __builtin_bit_cast(bf16x8, (u32x4{m0[0], m0[1], m1[0], m1[1]})),
                __builtin_bit_cast(bf16x8, (u32x4{l0[0], l0[1], l1[0], l1[1]}))};

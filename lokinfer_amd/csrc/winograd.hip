@@ -220,7 +220,7 @@ __global__ __launch_bounds__(256, 3) void winoMmKernel(WinoMmArgs p) {
 #pragma unroll
     for (int i = 0; i < S; ++i) {
       u32x2 h, m, l;
-      split3(ra.v[i], h, m, l);
+      split3(ra.v[i], kSplitScale, h, m, l);
       const int s2 = 4 * srow + 2 * ((squad >> 1) ^ ((srow >> 3) & 1)) + (squad & 1);
       reinterpret_cast<u32x2*>(As[i][0])[s2] = h;
       reinterpret_cast<u32x2*>(As[i][1])[s2] = m;
@@ -228,7 +228,7 @@ __global__ __launch_bounds__(256, 3) void winoMmKernel(WinoMmArgs p) {
     }
     if constexpr (N > 1) {
       unsigned h, m, l;
-      split3(ra.x, 0.0f, h, m, l);
+      split3(ra.x, 0.0f, kSplitScale, h, m, l);
       const int s8 = 8 * (xrow * 2 + ((xch >> 3) ^ ((xrow >> 3) & 1))) + (xch & 7);
       reinterpret_cast<unsigned short*>(As[xsub][0])[s8] = static_cast<unsigned short>(h);
       reinterpret_cast<unsigned short*>(As[xsub][1])[s8] = static_cast<unsigned short>(m);
@@ -254,7 +254,7 @@ __global__ __launch_bounds__(256, 3) void winoMmKernel(WinoMmArgs p) {
       return Frag3{__builtin_bit_cast(bf16x8, r[0]), __builtin_bit_cast(bf16x8, r[1]),
                    __builtin_bit_cast(bf16x8, r[2])};
     else
-      return split3(r[0], r[1]);
+      return split3(r[0], r[1], kSplitScale);
   };
 
   f32x16 acc;
