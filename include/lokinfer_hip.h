@@ -267,7 +267,8 @@ int lk_hip_wino_adain_affine_lc_f32(const float* stats, const float* gb, float* 
 
 /* ---- f32 GEMM over split weights (MI355X backend): the weight in three exact bf16 parts, laid out once in
  *      matrix-fragment order, the products on the bf16 matrix cores at f32 precision ---- */
-/* w f32[K, N] (nt = 0) or f32[N, K] (nt = 1) -> ws, ceil(N / 32) ceil(K / 16) 3072 bytes (parts of every float, as us) */
+/* w f32[K, N] (nt = 0) or f32[N, K] (nt = 1) -> ws, ceil(N / 32) ceil(K / 16) 3072 bytes: the parts of
+ * 2^23 W (an element of 2^105 and above, whose parts would pass the largest float, is a NaN part and its own bits) */
 int lk_hip_split_weight_f32(const float* w, void* ws, int64_t n, int64_t k, int nt, void* stream);
 /* out[M, N] = (act(a[M, K] W + bias) + res) * scale (act 0 none, 1 ReLU, 2 gelu_tanh; bias, res optional); K % 8 == 0,
  * a and ws 16-byte aligned */

@@ -42,7 +42,7 @@ __global__ __launch_bounds__(256) void splitWeightKernel(const float* __restrict
 #pragma unroll
     for (int e = 0; e < 8; ++e) v[e] = col < n && k0 + e < k ? w[nt ? col * k + k0 + e : (k0 + e) * n + col] : 0.0f;
     u32x4 parts[3];
-    splitExact(v, parts);
+    splitExact(v, kSplitScale, parts);
 #pragma unroll
     for (int q = 0; q < 3; ++q) ws[(nb * kb + kc) * 192 + q * 64 + lane] = parts[q];
   }
@@ -194,7 +194,7 @@ __global__ __launch_bounds__(64 * NW * KG) void gemmWsKernel(GemmWsParams p) {
   for (int i = 0; i < TM; ++i)
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-      acc[i][r] = (acc[i][r] + low[i][r]) * kSplitUnscale;
+      acc[i][r] = (acc[i][r] + low[i][r]) * (kSplitUnscale * kSplitUnscale);
       bad = fmaf(acc[i][r], 0.0f, bad);  // NaN after either
     }
   if (__any(bad != bad)) {
@@ -207,7 +207,7 @@ __global__ __launch_bounds__(64 * NW * KG) void gemmWsKernel(GemmWsParams p) {
       f32x4 b[3];
 #pragma unroll
       for (int q = 0; q < 3; ++q) b[q] = __builtin_bit_cast(f32x4, wb[static_cast<int64_t>(c) * 192 + q * 64]);
-      joinParts(b);
+      joinParts(b, kSplitUnscale);
 #pragma unroll
       for (int i = 0; i < TM; ++i) {
         const float* ar = p.a + min<int64_t>(m0 + 32 * i + lr, lastRow) * p.k;

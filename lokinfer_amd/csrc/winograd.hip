@@ -352,7 +352,7 @@ __global__ __launch_bounds__(256, 3) void winoMmKernel(WinoMmArgs p) {
       for (int e = 0; e < E; ++e) {
         RawB bq;
         loadB(uf, e, bq);
-        if constexpr (UL == 2) joinParts(bq);
+        if constexpr (UL == 2) joinParts(bq, 1.0f);
         const float* vr = vf + vRow(arow + e % N) + 16 * (e / N) + 8 * lk;
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
@@ -480,7 +480,7 @@ __global__ __launch_bounds__(256) void winoSplitUKernel(const float* __restrict_
 #pragma unroll
     for (int k = 0; k < 8; ++k) v[k] = src[(k >> 2) * 256 + (k & 3)];
     u32x4 parts[3];
-    splitExact(v, parts);
+    splitExact(v, 1.0f, parts);
 #pragma unroll
     for (int q = 0; q < 3; ++q) us[((slab * 2 + half) * sets + set) * 192 + q * 64 + lane] = parts[q];
   }

@@ -135,17 +135,18 @@ def test_gemm_ws_small_operands(lk, m, k, n, planes, small):
 
 
 def test_split_weight_parts(lk):
-    """Every element is the sum of its parts, or, where three bf16 parts cannot hold it, stored whole behind a NaN."""
+    """2^23 times every element is the sum of its parts down to the smallest denormals; only one that the factor takes past
+    the largest float is stored whole behind a NaN (its columns leave the bf16 matrix cores)."""
     r = np.random.default_rng(9)
-    w = (r.standard_normal((64, 96)) * 2.0 ** r.integers(-149, 100, (64, 96))).astype(np.float32)
-    w[0, :4] = [0.0, -0.0, 2.0 ** -149, -(2.0 ** -110 - 2.0 ** -134)]
+    w = (r.standard_normal((64, 96)) * 2.0 ** r.integers(-149, 125, (64, 96))).astype(np.float32)
+    w[0, :8] = [0.0, -0.0, 2.0 ** -149, -(2.0 ** -110 - 2.0 ** -134), 3.4028235e38, 2.0 ** 105, np.inf, -(2.0 ** 105 - 2.0 ** 81)]
     p = lk.ops.split_weight(G(lk, w)).ws.numpy().view(np.uint16).reshape(3, 4, 3, 2, 32, 8).astype(np.uint32)
     p = p.transpose(2, 1, 3, 5, 0, 4).reshape(3, 64, 96)  # part, (chunk, half, k), (block, column)
     f = (p << 16).view(np.float32)
     whole = np.isnan(f[0])
-    assert whole.any() and (np.abs(w[whole]) < 2.0 ** -110).all()
+    assert np.array_equal(whole, np.isfinite(w) & (np.abs(w) >= 2.0 ** 105))
     with np.errstate(invalid="ignore"):
-        back = np.where(whole, (p[1] << 16 | p[2]).view(np.float32), (f[0] + f[1]) + f[2])
+        back = np.where(whole, (p[1] << 16 | p[2]).view(np.float32), ((f[0] + f[1]) + f[2]) * np.float32(2.0 ** -23))
     assert np.array_equal(back, w)
 
 
