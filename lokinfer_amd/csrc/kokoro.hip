@@ -368,9 +368,10 @@ namespace lkh {
 int residueStats(const float* x, float* st, int64_t l, int64_t c, int d, int64_t chunks, hipStream_t s) {
   if (l <= 0 || c <= 0 || d < 1 || chunks < 1) return 1;
   dim3 grid(static_cast<unsigned>(ceilDiv(c, 64)), static_cast<unsigned>(d * chunks));
-  // short loads per thread while a block's latency is what the launch takes, long ones where it streams: G = 4 / 8 at
-  // 287 x 1024 4.8 / 3.8 us, 5740 x 256 4.9 / 3.9, 34441 x 128 5.4 / 5.2, 293281 x 128 26.4 / 28.1
-  if (static_cast<int64_t>(grid.x) * grid.y < 2048)
+  // short loads per thread while a block's latency is what the launch takes, up to some three blocks per CU, long ones where
+  // it streams: G = 4 / 8 at 287 x 1024 4.6 / 3.6 us, 5740 x 256 4.6 / 3.6, 34441 x 128 (540 blocks) 5.1 / 4.8, 20000 x 256
+  // (628) 5.2 / 5.0, 25000 x 256 (784) 5.4 / 5.6, 48880 x 256 10.4 / 11.6, 293281 x 128 25.8 / 27.5
+  if (static_cast<int64_t>(grid.x) * grid.y < 700)
     hipLaunchKernelGGL(lkd::statsKernel<8>, grid, dim3(512), 0, s, x, st, l, c, d, chunks);
   else
     hipLaunchKernelGGL(lkd::statsKernel<4>, grid, dim3(256), 0, s, x, st, l, c, d, chunks);
