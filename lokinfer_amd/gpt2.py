@@ -155,6 +155,8 @@ class Gpt2Generator(Gpt2Decoder):
         self.sk = tuple(sk)
         dev = self.w["transformer.wte.weight"].t.device
         self.positions = torch.arange(N_POS, dtype=torch.int64, device=dev)  # device pos views, no host copies
+        self.split_keys = [k for k in self.w if k.endswith(("attn.c_attn.weight", "attn.c_proj.weight", "mlp.c_fc.weight",
+                                                            "mlp.c_proj.weight"))]
         self.ws: dict[str, ops.SplitWeight] = {}
         self._laid: dict[str, tuple] = {}  # the torch tensor behind each split weight and its version when laid out
         self.split_weights()
@@ -164,9 +166,8 @@ class Gpt2Generator(Gpt2Decoder):
         """Lays the chunk forward's split weights out from `w`: all of them, or those written since the last time."""
         capturing = torch.cuda.is_current_stream_capturing()
         laid_out = False
-        for k, v in self.w.items():
-            if not k.endswith(("attn.c_attn.weight", "attn.c_proj.weight", "mlp.c_fc.weight", "mlp.c_proj.weight")):
-                continue
+        for k in self.split_keys:
+            v = self.w[k]
             version = None if v.t.is_inference() else v.t._version  # an inference tensor has no count: laid out anew
             laid = self._laid.get(k)
             if written_only and laid is not None and laid[0] is v.t and version is not None and laid[1] == version:
@@ -186,10 +187,13 @@ class Gpt2Generator(Gpt2Decoder):
         h = ops.embedding2_add_f32_gpu(w[P + "wte.weight"], ids, w[P + "wpe.weight"], pids)
         ln = ops.layernorm_f32_gpu(h, w[P + "h.0.ln_1.weight"], w[P + "h.0.ln_1.bias"], eps=LN_EPS)
 
+        for k, s in zip((D, FFN), self.sk):
+            if s:
+                ops.check_splits(k, s)
+        splits_of = [s if s and ops.splitk_planes(T, D, s) > 1 else 0 for s in self.sk]
+
         def proj_ln(x, wk, res, ln_key, splits):  # (res + x @ W + b, LN of it)
             if splits:
-                ops.check_splits(x.shape[1], splits)
-            if splits and ops.splitk_planes(T, D, splits) > 1:
                 parts = ops.gemm_ws_splitk_f32_gpu(x, self.ws[wk + "weight"], splits)
                 return ops.add_bias_layernorm2_sk_f32_gpu(parts, w[wk + "bias"], res, w[ln_key + "weight"],
                                                           w[ln_key + "bias"], eps=LN_EPS)
@@ -201,9 +205,9 @@ class Gpt2Generator(Gpt2Decoder):
             nxt = f"{P}h.{i + 1}.ln_1." if i + 1 < N_LAYER else P + "ln_f."
             qkv = ops.gemm_ws_f32_gpu(ln, self.ws[L + "attn.c_attn.weight"])
             att = ops.attention_gen2_f32_gpu(qkv, kc, vc, pos, w[L + "attn.c_attn.bias"], heads=HEADS)
-            h, ln = proj_ln(att, L + "attn.c_proj.", h, L + "ln_2.", self.sk[0])
+            h, ln = proj_ln(att, L + "attn.c_proj.", h, L + "ln_2.", splits_of[0])
             f = ops.gemm_ws_f32_gpu(ln, self.ws[L + "mlp.c_fc.weight"], w[L + "mlp.c_fc.bias"], act="gelu")
-            h, ln = proj_ln(f, L + "mlp.c_proj.", h, nxt, self.sk[1])
+            h, ln = proj_ln(f, L + "mlp.c_proj.", h, nxt, splits_of[1])
         logits = ops.gemm_nt_f32_gpu_mps(ops.view(ln, [1, D], offset=(T - 1) * D), w[P + "wte.weight"])
         return logits, ops.argmax_f32_gpu(logits)
 

@@ -264,7 +264,7 @@ def gemm_ws_f32_gpu(a, w: SplitWeight, bias=None, act="none", residual=None):
     """(MI355X backend) act(a f32[M, K] @ w + bias) [+ residual] with f32 precision on the bf16 matrix cores, as
     gemm_steel_f32_gpu over a plain weight; K % 8 == 0."""
     _f32(a, rank=2)
-    check(a.shape[1] == w.shape[0], f"gemm_ws: inner dims differ: {a.shape}, {w.shape}")
+    check(a.shape[1] == w.shape[0], "gemm_ws: inner dims differ")
     check(a.shape[1] % 8 == 0, "K must be a multiple of 8")
     s = (a.shape[0], w.shape[1])
     if bias is None:
@@ -282,7 +282,7 @@ def gemm_ws_splitk_f32_gpu(a, w: SplitWeight, splits):
     """(MI355X backend) gemm_splitk_f32_gpu over a split weight: partials f32[S, M, N] (rule splitk_planes) for
     add_bias_layernorm2_sk_f32_gpu. For few rows and a long K, whose one-launch sum leaves CUs idle."""
     _f32(a, rank=2)
-    check(a.shape[1] == w.shape[0] and a.shape[1] % 8 == 0, f"gemm_ws: a f32[M, K], K % 8 == 0: {a.shape}, {w.shape}")
+    check(a.shape[1] == w.shape[0] and a.shape[1] % 8 == 0, "gemm_ws: a f32[M, K] of the weight's K, a multiple of 8")
     check(1 <= int(splits) <= 64, "splits must be 1 .. 64")
     return _launch("gemm_ws_splitk_f32_gpu", [a, w.ws], [(int(splits), a.shape[0], w.shape[1])], dict(splits=int(splits)))
 
