@@ -279,32 +279,33 @@ class KokoroGpu:
         M = "bert.encoder.embedding_hidden_mapping_in"
         h = ops.gemm_bias_f32_gpu(e, self.g(M + ".weight", _t), self.g(M + ".bias"))
         L = "bert.encoder.albert_layer_groups.0.albert_layers.0."
-        wqkv = self.split_w("albert#wqkv", lambda: np.concatenate(
-            [self.sd[L + f"attention.{n}.weight"] for n in ("query", "key", "value")], axis=0))
+
+        def qkv_w():
+            return np.concatenate([self.sd[L + f"attention.{n}.weight"] for n in ("query", "key", "value")], axis=0)
+
         bqkv = self.const("albert#bqkv", lambda: np.concatenate(
             [self.sd[L + f"attention.{n}.bias"] for n in ("query", "key", "value")]))
+        # Up to 8 tokens q, k and v are row dots over the plain weight: in us, row dots / split-weight GEMM, 511 / 574 at 2
+        # tokens, 551 / 599 at 6, 593 / 600 at 8, 603 / 599 at 9 (where gemm_nt is a GEMM). Below 64 output tiles (T <= 320)
+        # the projections feeding a LayerNorm split K over workgroups too, their planes summed by it; the 768-deep one in
+        # one launch or two ranges: 670 / 651 at 32 tokens, 666 / 653 at 59, 945 / 944 at 320.
+        dots, sk = t <= 8, ops.splitk_planes(t, 768, 4) > 1
+        wqkv = self.const("albert#wqkv_nt", qkv_w) if dots else self.split_w("albert#wqkv", qkv_w)
 
-        # Below 64 output tiles (T <= 320) the FFN's 2048-deep output projection splits K over workgroups too, its planes
-        # summed by the LayerNorm
-        sk = ops.splitk_planes(t, 768, 4) > 1
+        def split(p):
+            return self.split_w(L + p, lambda: self.sd[L + p + ".weight"])
 
-        def linear(x, p, **kw):
-            return ops.gemm_ws_f32_gpu(x, self.split_w(L + p, lambda: self.sd[L + p + ".weight"]), **kw)
+        def proj_ln(x, res, p, ln, splits):
+            rest = (self.g(L + p + ".bias"), res, self.g(L + ln + ".weight"), self.g(L + ln + ".bias"))
+            if sk:
+                return ops.add_bias_layernorm2_sk_f32_gpu(ops.gemm_ws_splitk_f32_gpu(x, split(p), splits), *rest, eps=1e-12)[1]
+            return ops.add_bias_layernorm_f32_gpu(ops.gemm_ws_f32_gpu(x, split(p)), *rest, eps=1e-12)
 
         for _ in range(12):
-            a = ops.attention_qkv_sg_f32_gpu(ops.gemm_ws_f32_gpu(h, wqkv), bqkv, heads=12)
-            h = ops.add_bias_layernorm_f32_gpu(linear(a, "attention.dense"), self.g(L + "attention.dense.bias"), h,
-                                               self.g(L + "attention.LayerNorm.weight"),
-                                               self.g(L + "attention.LayerNorm.bias"), eps=1e-12)
-            f = linear(h, "ffn", bias=self.g(L + "ffn.bias"), act="gelu")
-            ln = (self.g(L + "ffn_output.bias"), h, self.g(L + "full_layer_layer_norm.weight"),
-                  self.g(L + "full_layer_layer_norm.bias"))
-            if sk:
-                parts = ops.gemm_ws_splitk_f32_gpu(f, self.split_w(L + "ffn_output", lambda: self.sd[L + "ffn_output.weight"]),
-                                                   4)
-                h = ops.add_bias_layernorm2_sk_f32_gpu(parts, *ln, eps=1e-12)[1]
-            else:
-                h = ops.add_bias_layernorm_f32_gpu(linear(f, "ffn_output"), *ln, eps=1e-12)
+            q = ops.gemm_nt_f32_gpu_mps(h, wqkv) if dots else ops.gemm_ws_f32_gpu(h, wqkv)
+            h = proj_ln(ops.attention_qkv_sg_f32_gpu(q, bqkv, heads=12), h, "attention.dense", "attention.LayerNorm", 2)
+            f = ops.gemm_ws_f32_gpu(h, split("ffn"), bias=self.g(L + "ffn.bias"), act="gelu")
+            h = proj_ln(f, h, "ffn_output", "full_layer_layer_norm", 4)
         return h
 
     def text_encoder_cnn(self, ids: Tensor) -> Tensor:
