@@ -46,14 +46,15 @@ def test_gemm_ws(lk, m, k, n):
     assert (np.abs(z - gelu) <= 1.2 * bound + 1e-6 * (1 + np.abs(x))).all()  # |gelu'| <= 1.13; f32 tanh
 
 
-@pytest.mark.parametrize("m,k,n", [(33, 40, 70), (200, 768, 64), (487, 768, 768), (8200, 64, 1056)])
-def test_gemm_ws_extreme_operands(lk, m, k, n):
+@pytest.mark.parametrize("m,k,n,planes", [s + (1,) for s in [(33, 40, 70), (200, 768, 64), (487, 768, 768), (8200, 64, 1056)] + KERNELS]
+                         + [(59, 256, 96, 4), (256, 136, 768, 4)])
+def test_gemm_ws_extreme_operands(lk, m, k, n, planes):
     """Infinities, NaN and values past the largest bf16 give what the f32 sum gives; rows of very different magnitude
-    keep f32's relative error each; a weight holding such values too."""
+    keep f32's relative error each; a weight holding such values too. Through every kernel, and the split-K planes."""
     r = np.random.default_rng(m + k + n)
     a = (r.standard_normal((m, k)) * 10.0 ** r.integers(-18, 18, (m, 1))).astype(np.float32)
     w = r.standard_normal((k, n)).astype(np.float32)
-    y = lk.ops.gemm_ws_f32_gpu(G(lk, a), lk.ops.split_weight(G(lk, w))).numpy()
+    y = _products(lk, a, w, planes)
     assert (np.abs(y - a.astype(np.float64) @ w) <= 2.0 ** -24 * (4 + np.sqrt(k)) * (np.abs(a).astype(np.float64) @ np.abs(w))).all()
     a = r.standard_normal((m, k)).astype(np.float32)
     for where in ("a", "w"):
@@ -67,7 +68,7 @@ def test_gemm_ws_extreme_operands(lk, m, k, n):
             with np.errstate(all="ignore"):
                 ref = x.astype(np.float64) @ v
                 bound = 2.0 ** -24 * (4 + np.sqrt(k)) * (np.abs(x).astype(np.float64) @ np.abs(v))  # f32 sums of k products
-            got = lk.ops.gemm_ws_f32_gpu(G(lk, x), lk.ops.split_weight(G(lk, v))).numpy()
+            got = _products(lk, x, v, planes)
             with np.errstate(all="ignore"):
                 fits = np.abs(ref) < 3e38
                 assert np.array_equal(np.isnan(ref), np.isnan(got))
@@ -98,7 +99,7 @@ def test_gemm_ws_refuses(lk):
 
 
 def _products(lk, a, w, planes):
-    """a w, by one launch or as the sum of `planes` K ranges (each entry of the tests that use it is one product)."""
+    """a w, by one launch or as the sum of `planes` K ranges."""
     ws = lk.ops.split_weight(G(lk, w))
     if planes == 1:
         return lk.ops.gemm_ws_f32_gpu(G(lk, a), ws).numpy()

@@ -326,7 +326,9 @@ def test_wino_mm_extreme_operands(gpu, ci, l, k, layout):
         big = np.abs(ref) > 3e38  # overflows in f32
         assert np.array_equal(np.isnan(ref), np.isnan(got))
         ok = np.isfinite(ref) & ~big
-        assert np.isfinite(got[ok]).all()
+        fine = np.where(np.isfinite(v), v, 0)  # what the finite outputs are sums of
+        mag = _mm_exact(np.abs(fine), np.abs(u), np.concatenate([tr[:a * a], at.ravel()]), l, k, a)
+        assert (np.abs(got[ok] - ref[ok]) <= 2.0 ** -24 * (6 + 2 * np.sqrt(n * ci * a)) * mag[ok]).all()
         inf = np.isinf(ref)
         assert np.array_equal(got[inf], ref[inf].astype(np.float32))
 
@@ -397,6 +399,30 @@ def test_wino_mm_small_operands(gpu, ci, l, k, tile, d, layout):
         assert (np.abs(run(tiny, u * big) - exact(tiny, u * big)) <= bound(tiny, u * big)).all()
     tiny = (u * 2.0 ** -r.integers(100, 148, 64)).astype(np.float32)
     assert (np.abs(run(v * big, tiny) - exact(v * big, tiny)) <= bound(v * big, tiny)).all()
+
+
+@pytest.mark.parametrize("layout", [0, 1, 2])
+@pytest.mark.parametrize("ci,l,k,tile,d", MM_KERNELS)
+def test_wino_mm_nonfinite_operands(gpu, ci, l, k, tile, d, layout):
+    """Infinities, NaN and values past the largest bf16, in V or in U, through every kernel: they reach the outputs that
+    the f32 sums take them to, and every finite output of the recomputed tiles is the f32 sum."""
+    run, v0, u0, exact, bound = _mm_operands(gpu, np.random.default_rng(ci + l + k), ci, l, k, tile, d, layout)
+    r1 = len(v0) // (d * len(u0))
+    for bad in (np.inf, -np.inf, np.nan, 3.4e38):
+        for where in ("v", "u"):
+            v, u = (v0, u0 * np.float32(0.15)) if where == "v" else (v0 * np.float32(0.15), u0)  # no product past 3.4e38
+            v, u = v.copy(), u.copy()
+            if where == "v":
+                v[r1 + 3, 5] = v[(len(u0) - 1) * r1 + 9, ci - 1] = bad
+            else:
+                u[1, 5, 7] = u[len(u0) - 1, ci - 1, 40] = bad
+            with np.errstate(all="ignore"):
+                ref, got = exact(v, u), run(v, u)
+                lim = bound(np.where(np.isfinite(v), v, 0), np.where(np.isfinite(u), u, 0))
+                assert np.array_equal(np.isnan(ref), np.isnan(got))
+                inf, ok = np.isinf(ref), np.abs(ref) < 3e38
+                assert np.array_equal(got[inf], ref[inf].astype(np.float32))
+                assert ok.any() and (np.abs(got[ok] - ref[ok]) <= lim[ok]).all()
 
 
 @pytest.mark.parametrize("layout", [0, 1, 2])
