@@ -27,11 +27,12 @@ struct GemmWsParams {
   int act;
   float scale;
   int planes;  // > 1: grid z = K range of an equal part of the steps, raw sums to c [planes, M, N]
+  float wUnscale;  // inverse of the factor that the parts of W carry
 };
 
 // One fragment's 8 values per thread; w [K, N] (nt 0) or [N, K] (nt 1).
 __global__ __launch_bounds__(256) void splitWeightKernel(const float* __restrict__ w, u32x4* __restrict__ ws, int64_t n,
-                                                        int64_t k, int nt) {
+                                                        int64_t k, int nt, float scale) {
   const int64_t kb = (k + 15) / 16, total = (n + 31) / 32 * kb * 64;
   for (int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < total;
        i += static_cast<int64_t>(gridDim.x) * blockDim.x) {
@@ -42,7 +43,7 @@ __global__ __launch_bounds__(256) void splitWeightKernel(const float* __restrict
 #pragma unroll
     for (int e = 0; e < 8; ++e) v[e] = col < n && k0 + e < k ? w[nt ? col * k + k0 + e : (k0 + e) * n + col] : 0.0f;
     u32x4 parts[3];
-    splitExact(v, kSplitScale, parts);
+    splitExact(v, scale, parts);
 #pragma unroll
     for (int q = 0; q < 3; ++q) ws[(nb * kb + kc) * 192 + q * 64 + lane] = parts[q];
   }
@@ -64,9 +65,6 @@ __global__ __launch_bounds__(64 * NW * KG) void gemmWsKernel(GemmWsParams p) {
   constexpr int UA = UNITS / TG;
   static_assert(UA >= 1 && UNITS % TG == 0, "whole A units per thread");
   using Stage = u32x4[KC][3][BM * 2];
-  struct Lds {
-    Stage a[2][KG];
-  };
   constexpr int RED = KG > 1 ? (KG - 1) * BM * 32 * NW * 4 : 16;
   constexpr int BYTES = sizeof(Stage) * KG > RED / 2 ? static_cast<int>(sizeof(Stage)) * KG : RED / 2;
   // two objects, so that the compiler sees that a step's stores and reads never meet; the reduction reuses both
@@ -194,7 +192,7 @@ __global__ __launch_bounds__(64 * NW * KG) void gemmWsKernel(GemmWsParams p) {
   for (int i = 0; i < TM; ++i)
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-      acc[i][r] = (acc[i][r] + low[i][r]) * (kSplitUnscale * kSplitUnscale);
+      acc[i][r] = (acc[i][r] + low[i][r]) * (kSplitUnscale * p.wUnscale);
       bad = fmaf(acc[i][r], 0.0f, bad);  // NaN after either
     }
   if (__any(bad != bad)) {
@@ -207,7 +205,7 @@ __global__ __launch_bounds__(64 * NW * KG) void gemmWsKernel(GemmWsParams p) {
       f32x4 b[3];
 #pragma unroll
       for (int q = 0; q < 3; ++q) b[q] = __builtin_bit_cast(f32x4, wb[static_cast<int64_t>(c) * 192 + q * 64]);
-      joinParts(b, kSplitUnscale);
+      joinParts(b, p.wUnscale);
 #pragma unroll
       for (int i = 0; i < TM; ++i) {
         const float* ar = p.a + min<int64_t>(m0 + 32 * i + lr, lastRow) * p.k;
@@ -273,27 +271,23 @@ __global__ __launch_bounds__(64 * NW * KG) void gemmWsKernel(GemmWsParams p) {
 
 }  // namespace lkd
 
-extern "C" {
+namespace {
 
-int lk_hip_split_weight_f32(const float* w, void* ws, int64_t n, int64_t k, int nt, void* stream) {
+int splitWeight(const float* w, void* ws, int64_t n, int64_t k, int nt, float scale, void* stream) {
   if (n < 0 || k < 0) return 1;
   if (n == 0 || k == 0) return 0;
   const int64_t total = (n + 31) / 32 * ((k + 15) / 16) * 64;
   hipLaunchKernelGGL(lkd::splitWeightKernel, dim3(static_cast<unsigned>(std::min<int64_t>((total + 255) / 256, 16384))),
-                     dim3(256), 0, static_cast<hipStream_t>(stream), w, static_cast<lkd::u32x4*>(ws), n, k, nt);
+                     dim3(256), 0, static_cast<hipStream_t>(stream), w, static_cast<lkd::u32x4*>(ws), n, k, nt, scale);
   return hipGetLastError() == hipSuccess ? 0 : 2;
 }
 
-}  // extern "C"
-
-namespace {
-
 int gemmWs(const float* a, const void* ws, const float* bias, const float* res, float* out, int64_t m, int64_t n,
-           int64_t k, int act, float scale, int planes, void* stream) {
+           int64_t k, int act, float scale, int planes, float wUnscale, void* stream) {
   if (m < 0 || n < 0 || k <= 0 || k % 8 != 0 || k > (int64_t{1} << 30)) return 1;
   if (((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(ws)) & 15) != 0) return 1;
   if (m == 0 || n == 0) return 0;
-  const lkd::GemmWsParams p{a, static_cast<const lkd::u32x4*>(ws), bias, res, out, m, n, k, act, scale, planes};
+  const lkd::GemmWsParams p{a, static_cast<const lkd::u32x4*>(ws), bias, res, out, m, n, k, act, scale, planes, wUnscale};
   hipStream_t s = static_cast<hipStream_t>(stream);
   const auto go = [&](auto kernel, int tm, int nw, int kg) {
     hipLaunchKernelGGL(kernel, dim3(lkh::ceilDiv(n, 32 * nw), lkh::ceilDiv(m, 32 * tm), static_cast<unsigned>(planes)),
@@ -342,15 +336,19 @@ int gemmWs(const float* a, const void* ws, const float* bias, const float* res, 
 
 extern "C" {
 
+int lk_hip_split_weight_f32(const float* w, void* ws, int64_t n, int64_t k, int nt, void* stream) {
+  return splitWeight(w, ws, n, k, nt, lkd::kSplitScale, stream);
+}
+
 int lk_hip_gemm_ws_f32(const float* a, const void* ws, const float* bias, const float* res, float* out, int64_t m,
                        int64_t n, int64_t k, int act, float scale, void* stream) {
-  return gemmWs(a, ws, bias, res, out, m, n, k, act, scale, 1, stream);
+  return gemmWs(a, ws, bias, res, out, m, n, k, act, scale, 1, lkd::kSplitUnscale, stream);
 }
 
 int lk_hip_gemm_ws_splitk_f32(const float* a, const void* ws, float* part, int64_t m, int64_t n, int64_t k, int planes,
                               void* stream) {
   if (planes < 1 || planes > 64) return 1;
-  return gemmWs(a, ws, nullptr, nullptr, part, m, n, k, 0, 1.0f, planes, stream);
+  return gemmWs(a, ws, nullptr, nullptr, part, m, n, k, 0, 1.0f, planes, lkd::kSplitUnscale, stream);
 }
 
 }  // extern "C"
@@ -359,17 +357,23 @@ namespace lkh {
 
 namespace {
 
-// split_weight_f32_gpu. ptrs: w, ws. ints: w(K, N) (nt: (N, K)), ws(ceil(N / 32), ceil(K / 16) 768), nt.
+// The kernels' attr `scaled`: 1, the parts of W are those of kSplitScale W. Graphs saved before it existed name none; their
+// weights are laid out, and read, unscaled.
+bool scaledAttr(const KernelArgs& a, uint32_t at) { return a.numInts > at && a.ints[at] == 1; }
+
+// split_weight_f32_gpu. ptrs: w, ws. ints: w(K, N) (nt: (N, K)), ws(ceil(N / 32), ceil(K / 16) 768), nt, [scaled].
 void runSplitWeight(ExecCtx& ctx, const KernelArgs& a) {
   const bool nt = a.ints[4] != 0;
   const int64_t k = a.ints[nt ? 1 : 0], n = a.ints[nt ? 0 : 1];
   LK_REQUIRE(ctx, a.ints[2] == (n + 31) / 32 && a.ints[3] == (k + 15) / 16 * 768,
              "split_weight: ws must be f32[ceil(N / 32), ceil(K / 16) 768]");
-  status(ctx, lk_hip_split_weight_f32(P<float>(a, 0), P<void>(a, 1), n, k, nt, ctx.stream), "split_weight: launch failed");
+  status(ctx,
+         splitWeight(P<float>(a, 0), P<void>(a, 1), n, k, nt, scaledAttr(a, 5) ? lkd::kSplitScale : 1.0f, ctx.stream),
+         "split_weight: launch failed");
 }
 
 // gemm_ws[_bias[_relu|_gelu|_res]]_f32_gpu. ptrs: a, ws, [bias], [res], out. ints: a(M, K), ws(..), [bias(N)],
-// [res(M, N)], out(M, N).
+// [res(M, N)], out(M, N), [scaled].
 template <bool BIAS, int ACT, bool RES>
 void runGemmWs(ExecCtx& ctx, const KernelArgs& a) {
   const int o = 4 + (BIAS ? 1 : 0) + (RES ? 2 : 0);
@@ -378,20 +382,23 @@ void runGemmWs(ExecCtx& ctx, const KernelArgs& a) {
              "gemm_ws: a f32[M, K], ws of an f32[K, N] weight, out f32[M, N]");
   const int outp = 2 + (BIAS ? 1 : 0) + (RES ? 1 : 0);
   status(ctx,
-         lk_hip_gemm_ws_f32(P<float>(a, 0), P<void>(a, 1), BIAS ? P<float>(a, 2) : nullptr,
-                            RES ? P<float>(a, 3) : nullptr, P<float>(a, outp), m, n, k, ACT, 1.0f, ctx.stream),
+         gemmWs(P<float>(a, 0), P<void>(a, 1), BIAS ? P<float>(a, 2) : nullptr, RES ? P<float>(a, 3) : nullptr,
+                P<float>(a, outp), m, n, k, ACT, 1.0f, 1, scaledAttr(a, o + 2) ? lkd::kSplitUnscale : 1.0f, ctx.stream),
          "gemm_ws: K must be a multiple of 8 and the operands 16-byte aligned");
 }
 
-// gemm_ws_splitk_f32_gpu. ptrs: a, ws, parts. ints: a(M, K), ws(..), parts(S, M, N): the first splitKPlanes planes hold
-// the K ranges' sums, as gemm_splitk's.
+// gemm_ws_splitk_f32_gpu. ptrs: a, ws, parts. ints: a(M, K), ws(..), parts(S, M, N), [scaled], splits: the first
+// splitKPlanes planes hold the K ranges' sums, as gemm_splitk's.
 void runGemmWsSplitK(ExecCtx& ctx, const KernelArgs& a) {
   const int64_t m = a.ints[0], k = a.ints[1], splits = a.ints[4], n = a.ints[6];
   LK_REQUIRE(ctx, a.ints[5] == m && a.ints[2] == (n + 31) / 32 && a.ints[3] == (k + 15) / 16 * 768 && splits >= 1,
              "gemm_ws_splitk: a f32[M, K], ws of an f32[K, N] weight, parts f32[S, M, N]");
-  status(ctx, lk_hip_gemm_ws_splitk_f32(P<float>(a, 0), P<void>(a, 1), P<float>(a, 2), m, n, k,
-                                        static_cast<int>(splitKPlanes(m, n, splits)), ctx.stream),
-         "gemm_ws_splitk: K must be a multiple of 8, S at most 64 and the operands 16-byte aligned");
+  const int64_t planes = splitKPlanes(m, n, splits);
+  LK_REQUIRE(ctx, planes <= 64, "gemm_ws_splitk: S must be at most 64");
+  const bool scaled = a.numInts > 8 && scaledAttr(a, 7);
+  status(ctx, gemmWs(P<float>(a, 0), P<void>(a, 1), nullptr, nullptr, P<float>(a, 2), m, n, k, 0, 1.0f,
+                     static_cast<int>(planes), scaled ? lkd::kSplitUnscale : 1.0f, ctx.stream),
+         "gemm_ws_splitk: K must be a multiple of 8 and the operands 16-byte aligned");
 }
 
 }  // namespace

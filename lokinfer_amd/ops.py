@@ -249,13 +249,16 @@ class SplitWeight:
         self.ws, self.shape = ws, tuple(shape)
 
 
+_SCALED = {"scaled": 1}  # the parts carry a factor of 2^23; graphs saved before the attr existed read unscaled ones
+
+
 def split_weight(w, nt: bool = False, out: SplitWeight | None = None) -> SplitWeight:
     """(MI355X backend) w f32[K, N] (nt: f32[N, K]) -> SplitWeight, laid out once for the gemm_ws ops; `out`: into
     that one's memory (a weight of the same shape, after it was written)."""
     _f32(w, rank=2)
     k, n = (w.shape[1], w.shape[0]) if nt else w.shape
     check(out is None or out.shape == (k, n), "out must be a SplitWeight of the same (K, N)")
-    ws = _launch("split_weight_f32_gpu", [w], [(-(-n // 32), -(-k // 16) * 768)], dict(nt=int(nt)),
+    ws = _launch("split_weight_f32_gpu", [w], [(-(-n // 32), -(-k // 16) * 768)], dict(nt=int(nt), scaled=1),
                  outs=None if out is None else [out.ws])
     return SplitWeight(ws, (k, n))
 
@@ -269,13 +272,13 @@ def gemm_ws_f32_gpu(a, w: SplitWeight, bias=None, act="none", residual=None):
     s = (a.shape[0], w.shape[1])
     if bias is None:
         check(act == "none" and residual is None, "act / residual need a bias")
-        return _launch("gemm_ws_f32_gpu", [a, w.ws], [s])
+        return _launch("gemm_ws_f32_gpu", [a, w.ws], [s], _SCALED)
     _bias_ok(bias, s[1])
     if residual is not None:
         check(act == "none" and tuple(residual.shape) == s, "residual must be f32[M, N], act none")
-        return _launch("gemm_ws_bias_res_f32_gpu", [a, w.ws, bias, residual], [s])
+        return _launch("gemm_ws_bias_res_f32_gpu", [a, w.ws, bias, residual], [s], _SCALED)
     name = {"none": "gemm_ws_bias_f32_gpu", "gelu": "gemm_ws_bias_gelu_f32_gpu", "relu": "gemm_ws_bias_relu_f32_gpu"}[act]
-    return _launch(name, [a, w.ws, bias], [s])
+    return _launch(name, [a, w.ws, bias], [s], _SCALED)
 
 
 def gemm_ws_splitk_f32_gpu(a, w: SplitWeight, splits):
@@ -284,7 +287,8 @@ def gemm_ws_splitk_f32_gpu(a, w: SplitWeight, splits):
     _f32(a, rank=2)
     check(a.shape[1] == w.shape[0] and a.shape[1] % 8 == 0, "gemm_ws: a f32[M, K] of the weight's K, a multiple of 8")
     check(1 <= int(splits) <= 64, "splits must be 1 .. 64")
-    return _launch("gemm_ws_splitk_f32_gpu", [a, w.ws], [(int(splits), a.shape[0], w.shape[1])], dict(splits=int(splits)))
+    return _launch("gemm_ws_splitk_f32_gpu", [a, w.ws], [(int(splits), a.shape[0], w.shape[1])],
+                   dict(splits=int(splits), scaled=1))
 
 
 # ---- conv1d (channel-last) ----------------------------------------------------------------------------------

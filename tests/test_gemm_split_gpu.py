@@ -159,3 +159,20 @@ def test_gemm_ws_nan_weights(lk, m, k, n):
     w.view(np.uint32)[1, 2], w.view(np.uint32)[k - 1, n - 1] = 0x7f800001, 0xff800001
     y = lk.ops.gemm_ws_f32_gpu(G(lk, a), lk.ops.split_weight(G(lk, w))).numpy()
     assert np.isnan(y[:, [2, n - 1]]).all() and np.isfinite(np.delete(y, [2, n - 1], 1)).all()
+
+
+def test_weights_of_earlier_graphs(lk):
+    """Kernels without the `scaled` attr (as saved graphs name them) lay out and read the parts of W itself: the same sums."""
+    r = np.random.default_rng(4)
+    m, k, n, s = 59, 256, 96, 4
+    a, w, b = (G(lk, r.standard_normal(x)) for x in ((m, k), (k, n), (n,)))
+    run, new = lk.ops._launch, lk.ops.split_weight(w)
+    old = run("split_weight_f32_gpu", [w], [new.ws.shape], dict(nt=0))
+    p = old.numpy().view(np.uint16).reshape(3, 16, 3, 2, 32, 8).astype(np.uint32).transpose(2, 1, 3, 5, 0, 4).reshape(3, k, n)
+    f = (p << 16).view(np.float32)
+    assert np.array_equal((f[0] + f[1]) + f[2], w.numpy())
+    for name, args, out, attrs, want in [
+            ("gemm_ws_f32_gpu", [a, old], (m, n), None, lk.ops.gemm_ws_f32_gpu(a, new)),
+            ("gemm_ws_bias_gelu_f32_gpu", [a, old, b], (m, n), None, lk.ops.gemm_ws_f32_gpu(a, new, b, act="gelu")),
+            ("gemm_ws_splitk_f32_gpu", [a, old], (s, m, n), dict(splits=s), lk.ops.gemm_ws_splitk_f32_gpu(a, new, s))]:
+        assert np.array_equal(run(name, args, [out], attrs).numpy(), want.numpy())
