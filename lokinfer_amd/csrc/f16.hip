@@ -776,7 +776,9 @@ __global__ __launch_bounds__(512) void gqaFlashKernel(GqaParams p) {
   for (int b = 0; b < 4; ++b)
 #pragma unroll
     for (int r = 0; r < 16; ++r) o[b][r] = 0.0f;
-  float m = -INFINITY, l = 0.0f;  // m in units of the raw score
+  // m: the running max times sc, rounded once and taken off everywhere as it is, so its rounding cancels between a query's
+  // weights, their sum, the corrections and the merge
+  float m = -INFINITY, l = 0.0f;
   const auto compute = [&](int tile, int b) {
     const h16* kt = sm + b * TILE + lr * FK_LD + 8 * lh;
     const h16* vt = sm + b * TILE + 32 * FK_LD + (4 * lh + ((lane >> 2) & 3)) * FV_LD + (lane & 16) + 4 * (lane & 3);
@@ -795,10 +797,10 @@ __global__ __launch_bounds__(512) void gqaFlashKernel(GqaParams p) {
     float mt = s[0];
 #pragma unroll
     for (int r = 1; r < 16; ++r) mt = fmaxf(mt, s[r]);
-    mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
+    mt = fmaxf(mt, __shfl_xor(mt, 32, 64)) * sc;
     if (__any(mt > m)) {  // some query's max grew
       const float mx = fmaxf(m, mt);
-      const float corr = mx == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f((m - mx) * sc);
+      const float corr = mx == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m - mx);
       l *= corr;
       m = mx;
 #pragma unroll
@@ -806,7 +808,7 @@ __global__ __launch_bounds__(512) void gqaFlashKernel(GqaParams p) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) o[bb][r] *= corr;
     }
-    const float mn = m == -INFINITY ? 0.0f : m * sc;  // no key up to here: nothing to add
+    const float mn = m == -INFINITY ? 0.0f : m;  // no key up to here: nothing to add
     float ls = 0.0f;
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
@@ -888,7 +890,7 @@ __global__ __launch_bounds__(512) void gqaFlashKernel(GqaParams p) {
 #pragma unroll
   for (int w = 0; w < NS; ++w) {
     const float lw = w < used ? lS[w * U + mu][q] : 0.0f;
-    scw[w] = lw == 0.0f ? 0.0f : __builtin_amdgcn_exp2f((mS[w * U + mu][q] - mxw) * sc);
+    scw[w] = lw == 0.0f ? 0.0f : __builtin_amdgcn_exp2f(mS[w * U + mu][q] - mxw);
     wsum += scw[w] * lw;
   }
   const float inv = 1.0f / wsum;

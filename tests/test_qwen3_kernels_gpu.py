@@ -309,3 +309,21 @@ def test_decode_fusions_equal_compositions(gpu, pos, cap):
     a = F.lm_head_last_opt_f16_gpu(F.rmsnorm_f16_gpu(G(lk, x), G(lk, g)), G(lk, tab)).numpy()
     b = F.rmsnorm_lm_head_last_opt_f16_gpu(G(lk, x), G(lk, g), G(lk, tab)).numpy()
     np.testing.assert_array_equal(a.view(np.uint32), b.view(np.uint32))
+
+
+@pytest.mark.parametrize("t", [100, 700, 2048])
+def test_attention_gqa_prefill_large_scores(gpu, t):
+    """Scores near 2^17, a step of 1 apart, rising and falling along the keys (exact in f32): the running maximum changes
+    from tile to tile and key group to key group, and its own rounding (2^-11 of a weight here) must not enter the weights.
+    Bound: the output's rounding to f16, and 2^-16 of the largest value for exp2, the f32 sums and the f16 pair of P."""
+    r = np.random.default_rng(t)
+    q = np.full((t, 16 * 128), 64.0, np.float16)
+    k = np.full((t, 8 * 128), 16.0, np.float16)
+    steps = (np.arange(t) * 7 % 61)  # of 2^-6, one ulp of 16
+    k[:, ::128] += (steps[:, None] * 2.0 ** -6).astype(np.float16)
+    v = r.standard_normal((t, 8 * 128)).astype(np.float16)
+    y = gpu.ops.f16_gpu.attention_gqa_f16_gpu(G(gpu, q), G(gpu, k), G(gpu, v), P(gpu, 0)).numpy().astype(np.float64)
+    w = np.exp((steps - steps.max()) * (64 * 2.0 ** -6 / np.sqrt(128)))  # the head's other dims add the same to every score
+    num = np.cumsum(w[:, None] * v.astype(np.float64), 0).reshape(t, 8, 128)
+    ref = np.repeat(num / np.cumsum(w)[:, None, None], 2, 1).reshape(t, 16 * 128)
+    assert (np.abs(y - ref) <= 2.0 ** -11 * np.abs(ref) + 2.0 ** -16 * np.abs(v).max()).all()
