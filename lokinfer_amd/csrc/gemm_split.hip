@@ -49,8 +49,10 @@ __global__ __launch_bounds__(256) void splitWeightKernel(const float* __restrict
   }
 }
 
-// Bound by L1 and issue rather than the MFMAs themselves (a 32 x 32 block reads 3 KB of B for 98 ns of MFMA): 1.3 to
-// 1.9 times the f32 MFMA kernels' rate; the six MFMAs alone would take 112 of the 258 us at (48880, 256, 1536).
+// Bound by what feeds the MFMAs: 1.1 to 2.3 times the f32 MFMA kernels' rate (the launcher's table, and 53 shapes of the
+// models' ranges). On the large tiles the matrix pipes are busy 46 - 49% of the time while waves wait to issue for half of
+// their cycles (A's conversion and LDS stores, 1.7 conflict cycles per LDS instruction, 3 KB of B for 98 ns of a 32 x 32
+// block's MFMAs); at (487, 768, 2304) they are busy 16%, at (59, 768, 2304) 3%, which is latency.
 //
 // Workgroup tile 32 TM rows x 32 NW columns; NW KG waves, wave (kg, wn) computing 32 TM x 32 over the K range of group kg
 // (the groups' partial tiles meet in LDS at the end, summed in order). A step is KS deep in every group: its A tile is

@@ -1,9 +1,11 @@
-// f32 products on the bf16 matrix cores. A float is the exact sum of three bf16 parts (8 + 8 + 8 significand bits):
+// f32 products on the bf16 matrix cores (the method of Henry, Tang and Heinecke, "Leveraging the bfloat16 Artificial
+// Intelligence Datatype For Higher-Precision Computations", 2019). A float is the exact sum of three bf16 parts (8 + 8 + 8
+// significand bits):
 // h = bf16(x), m = bf16(x - h), l = x - h - m, all rounded to nearest, so |m| <= 2^-8 |x| and |l| <= 2^-16 |x|. The
 // product of two such sums is nine bf16 products; the six of order up to 2^-16 are kept,
 //   x y = l h' + h l' + m m' + m h' + h m' + h h',
-// each exact in the f32 accumulator, and the dropped three (m l', l m', l l') are below 2^-23 |x y|, 2^-26 on average
-// and of either sign. Six 32x32x16 bf16 MFMAs take 192 cycles for 16 k where eight 32x32x2 f32 MFMAs take 512, and
+// each exact in the f32 accumulator, and the dropped three (m l', l m', l l') are about 2^-23 |x y| at most (their
+// bounds add up to (1 + 2^-9) 2^-23), 2^-26 on average and of either sign. Six 32x32x16 bf16 MFMAs take 192 cycles for 16 k where eight 32x32x2 f32 MFMAs take 512, and
 // they round the accumulator six times per 16 k instead of eight: against float64, 32 x 32 dot products of N(0, 1)
 // values are off by 1.6e-7 / 4.3e-7 / 9.5e-7 (2-norm) at K = 128 / 768 / 3072, on f32 MFMAs by 2.1e-7 / 4.9e-7 / 1.0e-6.
 //
@@ -81,7 +83,7 @@ __device__ __forceinline__ f32x16 mfma3(const Frag3& a, const Frag3& b, f32x16 a
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.h, b.h, acc, 0, 0, 0);
 }
 
-// The same in two accumulators, the h h' products in hi and the five smaller ones, at most 2^-7 of it, in lo: hi is rounded
+// The same in two accumulators, the h h' products in hi and the five smaller ones, about 2^-7 of it at most, in lo: hi is rounded
 // once per 16 k instead of six times (a third of the error at the same speed, for 16 more registers).
 __device__ __forceinline__ void mfma3(const Frag3& a, const Frag3& b, f32x16& hi, f32x16& lo) {
   lo = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.l, b.h, lo, 0, 0, 0);

@@ -138,11 +138,11 @@ struct WinoMmArgs {
 // banks. B bypasses LDS: a wave's fragment (16 k x 32 columns) comes straight from U, one step ahead, in coalesced
 // 16-byte loads.
 //
-// Measured (U split, graph replay), against the f32 MFMA form of this kernel, which reached 110 of 157 TFLOP/s and could
-// not overlap its vector instructions with its MFMAs: L = 293281, 128 -> 128 channels, K = 11 d = 5 456 -> 333 us,
-// K = 7 d = 3 335 -> 249 us, K = 3 with residual 254 -> 161 us; L = 48880, 256 -> 256, K = 11 d = 3 304 -> 213 us; L =
-// 5740, 256 -> 256, K = 7 d = 3 64 -> 49 us. Without the V staging the first takes 269 us, without the U loads 301, with
-// neither 223, and its bf16 MFMAs alone 148 (2.05 PFLOP/s).
+// Measured (graph replay, one box; with statistics), the f32 MFMA form of this kernel over U tiled, which could not overlap
+// its vector instructions with its MFMAs, against this one over U split: L = 293281, 128 -> 128 channels, K = 11 d = 5 427,
+// 321 us (under the profiler 362), K = 7 d = 3 311, 251, K = 3 with residual 252, 163; L = 48880, 256 -> 256, K = 11 d = 3
+// 281, 207; L = 5740, 256 -> 256, K = 7 d = 3 65, 47; L = 287, 1104 -> 1024, K = 3 40, 34. Of the first, with parts taken
+// out: 269 without the V staging, 301 without the U loads, 148 its bf16 MFMAs alone (of 333 before V was scaled).
 //
 // UL, the layout of U:
 //   0  U [A, N Ci, Co]: eight 4-byte loads per fragment, split before its MFMAs;
