@@ -314,6 +314,9 @@ int gemmWs(const float* a, const void* ws, const float* bias, const float* res, 
   // One block of rows leaves most CUs without a workgroup and waits for W: four waves that load four steps ahead instead of
   // eight that load two, W from memory: (32, 768, 2304) 11.4 against 12.0, f32 10.9; (32, 3072, 768) in four ranges 18.1
   // against 18.8, f32 19.6; W in the caches 8.5 against 7.7, f32 10.1. Narrow W keeps the eight: (32, 768, 768) 11.9, 12.7.
+  // The 32 x 64 tiles take steps of 32 k for a long K in one range, for the same reason. Steps of 16 | 32, W from memory:
+  // (512, 3072, 768) 31.9 | 29.6, (512, 2048, 768) 22.5 | 21.7, (512, 768, 768) 11.6 | 11.7, (160, 3072, 768) in four ranges 12.8
+  // | 12.8; in the caches 25.0 | 26.5, 18.3 | 19.4, 10.1 | 10.8, 9.7 | 10.5. A GPT-2 chunk of 512 tokens 1561 | 1532.
   const int64_t rows = static_cast<int64_t>(lkh::ceilDiv(m, 32)) * planes;
   const int64_t g1 = rows * lkh::ceilDiv(n, 32), g2 = rows * lkh::ceilDiv(n, 64), g4 = rows * lkh::ceilDiv(n, 128);
   const int64_t g8 = static_cast<int64_t>(lkh::ceilDiv(m, 64)) * lkh::ceilDiv(n, 128) * planes;
@@ -321,6 +324,8 @@ int gemmWs(const float* a, const void* ws, const float* bias, const float* res, 
     go(lkd::gemmWsKernel<1, 1, 4, 16, 4>, 1, 1, 4);
   else if (g1 <= 256)
     go(lkd::gemmWsKernel<1, 1, 8, 16, 2>, 1, 1, 8);
+  else if (g2 <= 256 && planes == 1 && k >= 2560)
+    go(lkd::gemmWsKernel<1, 2, 4, 32, 2>, 1, 2, 4);
   else if (g2 <= 256)
     go(lkd::gemmWsKernel<1, 2, 4, 16, 2>, 1, 2, 4);
   else if (g4 <= 256)

@@ -19,10 +19,11 @@ def G(lk, a):
 # (M, K, N): ragged rows, columns and K tails, K shorter than the wave groups, single rows and columns
 SHAPES = [(1, 8, 1), (1, 16, 33), (31, 24, 32), (33, 40, 31), (59, 768, 2304), (200, 2048, 96), (487, 768, 768),
           (500, 72, 700), (487, 2056, 770), (1030, 136, 2100), (4100, 40, 2090), (8200, 256, 1056)]
-# one per kernel of the launcher's rule: 32 x 32 with K over eight and four waves, 32 x 64 over four and two wave
-# groups, 32 x 128 over two and one, 64 x 128; the second half with one step or none for some of the groups
-KERNELS = [(33, 776, 70), (31, 264, 2100), (487, 776, 768), (500, 136, 2304), (430, 264, 2300), (640, 48, 2990),
-           (1500, 72, 2304), (32, 16, 2080), (600, 8, 768), (1000, 24, 700), (700, 40, 1300)]
+# one per kernel of the launcher's rule: 32 x 32 with K over eight and four waves, 32 x 64 over four (steps of 16 and
+# 32 k) and two wave groups, 32 x 128 over two and one, 64 x 128; the second half with one step or none for some of the
+# groups
+KERNELS = [(33, 776, 70), (31, 264, 2100), (487, 776, 768), (430, 2568, 700), (500, 136, 2304),
+           (430, 264, 2300), (640, 48, 2990), (1500, 72, 2304), (32, 16, 2080), (600, 8, 768), (1000, 24, 700), (700, 40, 1300)]
 
 
 @pytest.mark.parametrize("m,k,n", SHAPES + KERNELS)
