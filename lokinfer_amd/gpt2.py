@@ -147,7 +147,7 @@ class Gpt2Generator(Gpt2Decoder):
     0.50 GB of f32 weights, which the decode step streams; a program that only ever steps single tokens can use
     Gpt2Decoder). The copy follows `w`: a chunk lays out again, in place, every weight that torch counts a write to (or
     that was replaced) since. Writes that torch does not count (through `.data`, or by another library's pointer) need
-    a `split_weights()` call of their own."""
+    a `split_weights()` call of their own; new memory under the same tensor (`.data = x`) is seen."""
 
     def __init__(self, sd: dict[str, np.ndarray], graph: bool = True, fused: bool = True, sk=(2, 4),
                  chunk_graph: bool = False):
@@ -158,7 +158,7 @@ class Gpt2Generator(Gpt2Decoder):
         self.split_keys = [k for k in self.w if k.endswith(("attn.c_attn.weight", "attn.c_proj.weight", "mlp.c_fc.weight",
                                                             "mlp.c_proj.weight"))]
         self.ws: dict[str, ops.SplitWeight] = {}
-        self._laid: dict[str, tuple] = {}  # the torch tensor behind each split weight and its version when laid out
+        self._laid: dict[str, tuple] = {}  # the tensor behind each split weight, its version and memory when laid out
         self.split_weights()
         self.chunk_model = lk_capture(self._chunk, graph=chunk_graph)
 
@@ -170,11 +170,11 @@ class Gpt2Generator(Gpt2Decoder):
             v = self.w[k]
             version = None if v.t.is_inference() else v.t._version  # an inference tensor has no count: laid out anew
             laid = self._laid.get(k)
-            if written_only and laid is not None and laid[0] is v.t and version is not None and laid[1] == version:
+            if written_only and laid is not None and laid[0] is v.t and version is not None and laid[1:] == (version, v.t.data_ptr()):
                 continue
             self.ws[k] = ops.split_weight(v, out=self.ws.get(k))
             # while a graph is captured the copy is only recorded: the next eager call still has to make it
-            self._laid[k] = (v.t, None if capturing else version)
+            self._laid[k] = (v.t, None if capturing else version, v.t.data_ptr())
             laid_out = True
         if laid_out and not capturing:  # like an uploaded weight: ready for every stream that may run first
             torch.cuda.current_stream().synchronize()

@@ -146,6 +146,20 @@ def test_chunks_follow_written_weights(setup, chunk_graph):
         assert np.array_equal(got, G.Gpt2Generator(new)(ids, 0)) and not np.array_equal(got, first)
 
 
+def test_chunks_follow_swapped_memory(setup):
+    """A weight whose tensor was given other memory (`.data = x`, which torch does not count as a write)."""
+    import torch
+
+    G, O, sd, m = setup
+    ids = np.random.default_rng(7).integers(0, G.VOCAB, 40).astype(np.int64)
+    model, new, k = G.Gpt2Generator(sd), dict(sd), "transformer.h.5.mlp.c_proj.weight"
+    first = model(ids, 0)
+    new[k] = new[k] * np.float32(1.5)
+    model.w[k].t.data = torch.from_numpy(new[k]).to(model.w[k].t.device)
+    got = model(ids, 0)
+    assert np.array_equal(got, G.Gpt2Generator(new)(ids, 0)) and not np.array_equal(got, first)
+
+
 def test_split_weights_ready_on_any_stream(setup, monkeypatch):
     """A model built on one stream, where laying a weight out takes long, runs at once on another."""
     import torch
